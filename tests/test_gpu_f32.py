@@ -61,6 +61,25 @@ def test_f32_decode_matches_reference(Q, name):
         ref.close()
 
 
+@pytest.mark.parametrize("K", [64, 65, 79, 511, 512, 513, 575, 576, 640, 1023, 1087])
+def test_f32_gemv_group_edges_match_oracle(Q, K):
+    """The fp32 GEMV where its loop changes form: inputs around whole groups of 64
+    k rows, around the eight groups in flight (512) and around tiles of 16, with
+    a partial column panel: bit for bit against the oracle."""
+    cfg = [33, 48, 1, 3, 1, 16, K, 16]
+    ref = O.FModel(cfg, 10000.0, seed=K)
+    try:
+        g = gpu_model(Q, ref, cfg, 10000.0)
+        try:
+            for t in [1, 5, 32]:
+                r = ref.step(t).copy()
+                assert np.array_equal(bits(g.step(t)), bits(r)), (K, t)
+        finally:
+            g.close()
+    finally:
+        ref.close()
+
+
 @pytest.mark.parametrize("shape", [(4096, 4096), (14336, 4096), (4096, 1024), (300, 17), (1000, 130), (129, 16)])
 def test_f32_gemv_rows_match_oracle(Q, shape):
     """The fp32 GEMV at (K, N) through a one-layer model whose down projection
