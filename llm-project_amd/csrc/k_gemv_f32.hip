@@ -15,6 +15,8 @@
 // columns) sit 4, 8 and 12 lanes up, where a DPP row shift reaches them.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "qdev_math.h"
 #include "qdev_norm.h"
 #include "qhip.h"
@@ -246,107 +248,183 @@ __global__ void k_swiglu_f32(const float *gu, int dff, float *h) {
 
 // ---------------------------------------------------------------------------
 // Many-row f32 matmul (matrix.c:178-190 over M rows): the GEMMs of the batched
-// forward.  Every output element is one serial chain in k order, the
-// reference's, with each product rounded before its add.  A 64 x 64 block tile
-// gives each of 256 threads 4 rows x 4 columns, 16 independent chains; K is
-// staged kKT rows at a time through LDS (A transposed to [k][row], W from the
-// block's four panels as [k][column]), and the next stage's global loads are in
-// flight while the current one is summed.  A chain takes exactly K terms: a
-// padded 0 * w term would turn a -0 sum into +0.
+// forward.  Every output element is one serial chain in k order, the reference's,
+// with each product rounded before its add: a v_mul_f32 and a v_add_f32 a k row.
+//
+// A lane owns one column and R rows, a wave 64 columns (four panels), a block of
+// eight waves 8 * R rows of the same columns.  A row's value at a k row is the
+// same for the whole wave, so it comes through the scalar cache into SGPRs and is
+// the multiply's scalar operand: it costs no vector register, no LDS read and no
+// vector issue slot.  For that A is first packed by groups of R rows,
+// [ceil(M/R)][K][R], so that a wave reads one contiguous stream (R = 1: A itself).
+// W goes through LDS, 32 k rows a stage in two buffers with two more stages in
+// flight in registers, and a lane reads four k rows of its column at a time.
+// Bound: the VALU, two instructions a multiply-add without FMA (65 T lane-ops/s
+// reached by multiplies and adds alone), where eight waves a SIMD cover the scalar
+// loads; the loads' latency where a narrow output leaves fewer.  512 rows: K = 2048,
+// N = 16384 814 -> 626 us (54.9 TFLOP/s), N = 32000 1522 -> 1230, N = 3072
+// 264 -> 134; K = 8192, N = 2048 960 -> 377 (45.6), against 64 x 64 tiles of
+// 4 x 4 sums a thread with both operands read from LDS.
 // ---------------------------------------------------------------------------
-constexpr int kMT = 64;           // rows per block tile
-constexpr int kNT = 4 * kFC;      // columns per block tile: four panels
-constexpr int kKT = 32;           // k rows per LDS stage
-constexpr int kAS = kMT + 4;      // LDS stride of a k row of A
-constexpr int kWS = kNT + 4;      // LDS stride of a k row of W
+constexpr int kGW = 8;            // waves per block
+constexpr int kGN = 64;           // columns per block: four panels
+constexpr int kGK = 2 * kFK;      // k rows per LDS stage
 
-template <int MODE>
-__global__ __launch_bounds__(256) void k_gemm_f32(const float *A, int M, int K, const float *W, int N, float *out,
-                                                  const float *bias) {
-  __shared__ __align__(16) float As[kKT * kAS];
-  __shared__ __align__(16) float Ws[kKT * kWS];
-  const int tid = threadIdx.x;
-  const int i0 = blockIdx.y * kMT, j0 = blockIdx.x * kNT;
-  const int np = (N + kFC - 1) / kFC, kt = (K + kFK - 1) / kFK;
-  const bool vec = (K & 3) == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;   // whole aligned float4s
-  // staging of A: thread -> row ar, k offsets ak .. ak+7 of the stage
-  const int ar = tid >> 2, ak = (tid & 3) * 8;
-  const bool arow = i0 + ar < M;
-  const float *Ar = A + (size_t)(arow ? i0 + ar : 0) * K;
-  // staging of W: float4 f = tid + 256 g is panel f / 128, tile (f % 128) / 64, lane part f % 64 of the tile
-  float av[8];
-  float4 wv[2];
-  auto gload = [&](int k0) {
-    if (vec) {
+// rows of A -> groups of R rows, k rows outermost within a group (rows past M zero)
+template <int R>
+__global__ __launch_bounds__(256) void k_pack_rows(const float *A, int M, int K, float *P) {
+  const int k = blockIdx.x * 256 + threadIdx.x, i0 = blockIdx.y * R;
+  if (k >= K) return;
+  float v[R];
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int k = k0 + ak + 4 * h;
-        const float4 v = arow && k < K ? *reinterpret_cast<const float4 *>(Ar + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-        av[4 * h] = v.x; av[4 * h + 1] = v.y; av[4 * h + 2] = v.z; av[4 * h + 3] = v.w;
+  for (int r = 0; r < R; r++) v[r] = i0 + r < M ? A[(size_t)(i0 + r) * K + k] : 0.0f;
+  float *o = P + ((size_t)blockIdx.y * K + k) * R;
+#pragma unroll
+  for (int r = 0; r < R; r++) o[r] = v[r];
+}
+
+// N floats from a wave-uniform address, into SGPRs
+template <int N>
+struct SRow { typedef float V __attribute__((ext_vector_type(N), aligned(4))); };
+
+template <int MODE, int R>
+__global__ __launch_bounds__(64 * kGW) void k_gemm_f32(const float *Ap, int M, int K, const float *W, int N, float *out,
+                                                      const float *bias, int mt, int nt) {
+  constexpr int KB = R >= 8 ? 4 : 8, QB = KB / 4;     // k rows of a scalar batch
+  typedef typename SRow<R * KB>::V Batch;
+  typedef const __attribute__((address_space(4))) Batch *BatchPtr;
+  typedef const __attribute__((address_space(4))) float *ScalarPtr;
+  __shared__ float4 ws[2][kGK * kGN / 4];
+  const int b8 = blockIdx.x >> 3, mtile = b8 % mt, ntile = 8 * (b8 / mt) + (blockIdx.x & 7);
+  if (ntile >= nt) return;                            // uniform for the block
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i0 = (mtile * kGW + wave) * R, np = (N + kFC - 1) / kFC, kt = (K + kFK - 1) / kFK;
+  const bool work = i0 < M;                           // a wave past the last row only helps to stage
+  // staging: float4 tid of a stage is panel tid / 128, tile (tid / 64) % 2, part l of the tile; part
+  // l = 16*a + 4*s + b goes to slot 16*a + 4*(s ^ a) + b, so that the 16 columns of a panel, read at
+  // one s, fall in distinct banks
+  const int l = lane, pnl = ntile * 4 + (tid >> 7), tsub = (tid >> 6) & 1;
+  const int wslot = (tid & ~63) + (l & 48) + 4 * (((l >> 2) & 3) ^ (l >> 4)) + (l & 3);
+  const float4 *Wl = reinterpret_cast<const float4 *>(W) + ((size_t)min(pnl, np - 1) * kt) * (kFTile / 4) + l;
+  auto gload = [&](int st) __attribute__((always_inline)) {
+    return Wl[(size_t)min(2 * st + tsub, kt - 1) * (kFTile / 4)];     // past the last tile or panel: staged, never summed or stored
+  };
+  // this lane's column: slot of k rows 4*s .. +3 of tile t of a stage
+  const int ca = (lane >> 2) & 3, cslot = (lane >> 4) * 128 + 16 * ca + (lane & 3);
+  int rslot[4];
+#pragma unroll
+  for (int s = 0; s < 4; s++) rslot[s] = cslot + 4 * (s ^ ca);
+  const ScalarPtr As = (ScalarPtr)(uintptr_t)(Ap + (size_t)(i0 / R) * K * R);
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) acc[r] = 0.0f;
+
+  Batch av[2];
+  float4 wv[2][QB];
+  // nb batches of KB k rows of the stage at k0, from LDS buffer buf; av[0] holds the first on entry and
+  // the next stage's first on exit
+  auto sum = [&](int buf, int k0, int nb) __attribute__((always_inline)) {
+    constexpr int NB = kGK / KB;
+    ScalarPtr p = As + (size_t)k0 * R;
+    // the batch after the last: the next stage's first, or (nothing follows) one this wave has read
+    ScalarPtr pn = k0 + (nb + 1) * KB <= K ? p + nb * KB * R : As;
+    auto wload = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < QB; i++) wv[u & 1][i] = ws[buf][rslot[(u * QB + i) & 3] + ((u * QB + i) >> 2) * 64];
+    };
+    wload(0);
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+      if (u < nb) {
+        // scalar loads return out of order, so a wait is for all of them: this batch's, requested a
+        // batch ago, before the next one's are requested
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        if (u + 1 < NB) wload(u + 1);
+        av[(u + 1) & 1] = *(BatchPtr)(u + 1 < NB && u + 1 < nb ? p + (u + 1) * KB * R : pn);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < KB; e++) {
+          const float4 w4 = wv[u & 1][e >> 2];
+          const float w = (e & 3) == 0 ? w4.x : (e & 3) == 1 ? w4.y : (e & 3) == 2 ? w4.z : w4.w;
+          float m[R];
+#pragma unroll
+          for (int r = 0; r < R; r++) m[r] = av[u & 1][e * R + r] * w;
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int r = 0; r < R; r++) acc[r] = acc[r] + m[r];
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; e++) av[e] = arow && k0 + ak + e < K ? Ar[k0 + ak + e] : 0.0f;
-    }
-#pragma unroll
-    for (int g = 0; g < 2; g++) {
-      const int f = tid + 256 * g, p = blockIdx.x * 4 + (f >> 7), t = k0 / kFK + ((f >> 6) & 1);
-      wv[g] = p < np && t < kt ? *reinterpret_cast<const float4 *>(W + ((size_t)p * kt + t) * kFTile + (f & 63) * 4)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
-  const int ty = tid >> 4, tx = tid & 15;
-  float acc[4][4];
+  // the wave's part of stage t of A, touched (one value a 128-byte line) so that its scalar loads find it in L2
+  const float *At = Ap + (size_t)(work ? i0 / R : 0) * K * R;
+  auto touch = [&](int t) __attribute__((always_inline)) {
+    return At[(unsigned)min(t * kGK * R + (lane & (R - 1)) * 32, K * R - 1)];
+  };
+
+  float4 g[2];
+  g[0] = gload(0);
+  g[1] = gload(1);
+  float pf = touch(1);
+  if (work && K >= KB) av[0] = *(BatchPtr)As;
+  ws[0][wslot] = g[0];
+  g[0] = gload(2);
+  qd::lds_sync();
+  const int nst = K / kGK;
+  auto stage = [&](auto par, int t) __attribute__((always_inline)) {   // stage t, parity par
+    constexpr int P = decltype(par)::value;
+    ws[P ^ 1][wslot] = g[P ^ 1];                      // that buffer was last read in stage t - 1
+    asm volatile("" ::"v"(pf));
+    pf = touch(t + 2);
+    g[P ^ 1] = gload(t + 3);
+    __builtin_amdgcn_sched_barrier(0);
+    if (work) sum(P, t * kGK, kGK / KB);
+    qd::lds_sync();
+  };
+  int t = 0;
+  for (; t + 2 <= nst; t += 2) {
+    stage(std::integral_constant<int, 0>(), t);
+    stage(std::integral_constant<int, 1>(), t + 1);
+  }
+  ws[1][wslot] = g[1];                                // t is even: buffer 0 holds stage t, and t + 1 is the last
+  for (; t * kGK < K; t++) {                          // a whole stage, a partial one, or both (a chain takes exactly K terms)
+    const int kn = min(kGK, K - t * kGK), nb = kn / KB, buf = t & 1;
+    if (buf) qd::lds_sync();
+    if (!work) continue;
+    sum(buf, t * kGK, nb);
+    for (int k = nb * KB; k < kn; k++) {
+      const float w = reinterpret_cast<const float *>(&ws[buf][cslot + 4 * (((k >> 2) & 3) ^ ca) + (k >> 4) * 64])[k & 3];
 #pragma unroll
-  for (int r = 0; r < 4; r++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) acc[r][c] = 0.0f;
-  gload(0);
-  for (int k0 = 0; k0 < K; k0 += kKT) {
-    __syncthreads();                              // the previous stage is summed
-#pragma unroll
-    for (int e = 0; e < 8; e++) As[(ak + e) * kAS + ar] = av[e];
-#pragma unroll
-    for (int g = 0; g < 2; g++) {
-      const int f = tid + 256 * g;
-      const int l = f & 63, k = ((f >> 6) & 1) * kFK + 4 * ((l >> 2) & 3), j = (f >> 7) * kFC + 4 * (l >> 4) + (l & 3);
-      Ws[k * kWS + j] = wv[g].x;
-      Ws[(k + 1) * kWS + j] = wv[g].y;
-      Ws[(k + 2) * kWS + j] = wv[g].z;
-      Ws[(k + 3) * kWS + j] = wv[g].w;
-    }
-    __syncthreads();
-    if (k0 + kKT < K) gload(k0 + kKT);
-    const int kn = min(kKT, K - k0);
-    auto step = [&](int kk) {
-      const float4 a = *reinterpret_cast<const float4 *>(&As[kk * kAS + ty * 4]);
-      const float4 w = *reinterpret_cast<const float4 *>(&Ws[kk * kWS + tx * 4]);
-      const float ar4[4] = {a.x, a.y, a.z, a.w}, wr4[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) acc[r][c] = acc[r][c] + ar4[r] * wr4[c];
-    };
-    if (kn == kKT) {
-#pragma unroll 8
-      for (int kk = 0; kk < kKT; kk++) step(kk);
-    } else {
-      for (int kk = 0; kk < kn; kk++) step(kk);
+      for (int r = 0; r < R; r++) acc[r] = acc[r] + As[(size_t)(t * kGK + k) * R + r] * w;
     }
   }
+  if (!work) return;
+  const int j = ntile * kGN + lane;
+  if (j >= N) return;
+  const float bj = MODE == FMODE_PLAIN && bias ? bias[j] : 0.0f;
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int i = i0 + ty * 4 + r;
-    if (i >= M) continue;
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const int j = j0 + tx * 4 + c;
-      if (j >= N) continue;
-      float *o = out + (size_t)i * N + j;
-      if (MODE == FMODE_RESID) *o = *o + acc[r][c];
-      else *o = bias ? acc[r][c] + bias[j] : acc[r][c];
-    }
+  for (int r = 0; r < R; r++) {
+    if (i0 + r >= M) break;
+    float *o = out + (size_t)(i0 + r) * N + j;
+    if (MODE == FMODE_RESID) *o = *o + acc[r];
+    else *o = bias ? acc[r] + bj : acc[r];
   }
+}
+
+template <int R>
+int launch_gemm(int mode, int cls, const float *A, int M, int K, const float *W, int N, float *out, const float *bias,
+                float *pack) {
+  const int mt = (M + kGW * R - 1) / (kGW * R), nt = (N + kGN - 1) / kGN;
+  const dim3 grid(8 * mt * ((nt + 7) / 8)), block(64 * kGW);
+  if (R > 1) {
+    QH_LAUNCH(cls, k_pack_rows<R>, dim3((K + 255) / 256, (M + R - 1) / R), dim3(256), 0, A, M, K, pack);
+    A = pack;
+  }
+  if (mode == 0) QH_LAUNCH(cls, (k_gemm_f32<FMODE_PLAIN, R>), grid, block, 0, A, M, K, W, N, out, bias, mt, nt);
+  else QH_LAUNCH(cls, (k_gemm_f32<FMODE_RESID, R>), grid, block, 0, A, M, K, W, N, out, bias, mt, nt);
+  return 0;
 }
 
 }  // namespace
@@ -410,12 +488,34 @@ extern "C" int qhip_embed_f32_rows(const float *wte, int dm, const int *ids, int
   return 0;
 }
 
+// Floats of qhip_gemm_f32's pack workspace.
+extern "C" size_t qhip_gemm_f32_pack(int M, int K) { return (size_t)((M + 7) / 8) * 8 * K; }
+
 extern "C" int qhip_gemm_f32(int mode, int cls, const float *A, int M, int K, const float *W, int N, float *out,
-                             const float *bias) {
-  if (M <= 0 || K <= 0 || N <= 0 || M > 65535 * kMT) return qh::fail_msg("gemm_f32: bad shape");
-  const dim3 grid((N + kNT - 1) / kNT, (M + kMT - 1) / kMT);
-  if (mode == 0) QH_LAUNCH(cls, k_gemm_f32<FMODE_PLAIN>, grid, dim3(256), 0, A, M, K, W, N, out, bias);
-  else if (mode == 1) QH_LAUNCH(cls, k_gemm_f32<FMODE_RESID>, grid, dim3(256), 0, A, M, K, W, N, out, bias);
-  else return qh::fail_msg("gemm_f32: bad mode");
-  return 0;
+                             const float *bias, float *pack) {
+  if (M <= 0 || K <= 0 || N <= 0) return qh::fail_msg("gemm_f32: bad shape");
+  if (mode != 0 && mode != 1) return qh::fail_msg("gemm_f32: bad mode");
+  // Rows per wave.  A CU spends R + 0.65 units (4.4 ns) a k row on each of its blocks (R multiply-add
+  // pairs, and the reads around them), but no less than a batch of scalar loads takes to come back,
+  // which only other waves can cover: with one block a CU at least 3.0, 3.5, 4.7 and 14 units for R = 1,
+  // 2, 4, 8.  The R of the least time, the largest of equals (W is then read by fewer blocks).
+  // Measured, us (K = 8192, N = 2048): 50 rows 110 134 177 306 for R = 1 2 4 8, 130 rows 183 185 189 451,
+  // 512 rows 513 423 377 529; (K = 2048, N = 16384) 512 rows 986 784 662 626.
+  static const int least[4] = {300, 350, 470, 1400};
+  const int cus = qh::num_cus() > 0 ? qh::num_cus() : 256, nt = (N + kGN - 1) / kGN;
+  int best = 1;
+  long long cost = 0;
+  for (int i = 0; i < 4; i++) {
+    const int R = 1 << i;
+    const long long blocks = (long long)((M + kGW * R - 1) / (kGW * R)) * nt;
+    long long c = ((blocks + cus - 1) / cus) * (100 * R + 65);
+    if (c < least[i]) c = least[i];
+    if (i == 0 || c <= cost) { best = R; cost = c; }
+  }
+  switch (best) {
+    case 1: return launch_gemm<1>(mode, cls, A, M, K, W, N, out, bias, pack);
+    case 2: return launch_gemm<2>(mode, cls, A, M, K, W, N, out, bias, pack);
+    case 4: return launch_gemm<4>(mode, cls, A, M, K, W, N, out, bias, pack);
+    default: return launch_gemm<8>(mode, cls, A, M, K, W, N, out, bias, pack);
+  }
 }

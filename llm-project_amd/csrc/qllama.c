@@ -1194,13 +1194,16 @@ static int fwd_run(const FDev *f, float rope_base, const int *ids, int n, float 
   const size_t o_h = FTAKE((size_t)R * f->dff), o_lg = FTAKE(R * V), o_kc = FTAKE(per), o_vc = FTAKE(per);
   const size_t o_ws = FTAKE(qhip_pf_attention_scratch(R, f->H, n));
   const size_t o_cos = FTAKE(own_rope ? (size_t)n * half : 1), o_sin = FTAKE(own_rope ? (size_t)n * half : 1);
+  int kmax = f->dm > f->qd ? f->dm : f->qd;
+  if (f->dff > kmax) kmax = f->dff;
+  const size_t o_pk = FTAKE(qhip_gemm_f32_pack(R, kmax));
 #undef FTAKE
   uint8_t *b = (uint8_t*)qhip_malloc(off);
   if (!b) return 1;
   int *d_ids = (int*)(b + o_ids);
   float *X = (float*)(b + o_x), *xn = (float*)(b + o_xn), *qkv = (float*)(b + o_qkv), *q = (float*)(b + o_q);
   float *o = (float*)(b + o_o), *gu = (float*)(b + o_gu), *h = (float*)(b + o_h), *lg = (float*)(b + o_lg);
-  float *kc = (float*)(b + o_kc), *vc = (float*)(b + o_vc), *ws = (float*)(b + o_ws);
+  float *kc = (float*)(b + o_kc), *vc = (float*)(b + o_vc), *ws = (float*)(b + o_ws), *pk = (float*)(b + o_pk);
   const float *cs = f->rope_cos, *sn = f->rope_sin;
   int rc = qhip_h2d(d_ids, ids, (size_t)n * sizeof(int));
   if (!rc && own_rope) {        // positions past max_seq: tables of n rows (rope.c:58-61)
@@ -1213,19 +1216,19 @@ static int fwd_run(const FDev *f, float rope_base, const int *ids, int n, float 
       const int r = n - c0 < R ? n - c0 : R;
       float *Xc = X + (size_t)c0 * dm;
       rc |= qhip_rmsnorm_f32_rows(Xc, r, f->dm, f->g_attn[l], f->eps, xn);
-      rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->wqkv[l], f->nqkv, qkv, f->bqkv[l]);
+      rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->wqkv[l], f->nqkv, qkv, f->bqkv[l], pk);
       rc |= qhip_pf_rope_append(qkv, r, f->H, f->KVH, f->hd, cs, sn, c0, q, kc, vc, n);
       rc |= qhip_pf_attention(q, kc, vc, r, c0, f->H, f->KVH, f->hd, n, f->attn_scale, ws, o);
-      rc |= qhip_gemm_f32(1, FWD_CLS, o, r, f->qd, f->wo[l], f->dm, Xc, NULL);
+      rc |= qhip_gemm_f32(1, FWD_CLS, o, r, f->qd, f->wo[l], f->dm, Xc, NULL, pk);
       rc |= qhip_rmsnorm_f32_rows(Xc, r, f->dm, f->g_ffn[l], f->eps, xn);
-      rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->wgu[l], 2 * f->dff, gu, NULL);
+      rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->wgu[l], 2 * f->dff, gu, NULL, pk);
       rc |= qhip_swiglu_f32_rows(gu, r, f->dff, h);
-      rc |= qhip_gemm_f32(1, FWD_CLS, h, r, f->dff, f->wd[l], f->dm, Xc, NULL);
+      rc |= qhip_gemm_f32(1, FWD_CLS, h, r, f->dff, f->wd[l], f->dm, Xc, NULL, pk);
     }
   for (int c0 = 0; c0 < n && !rc; c0 += R) {   // final norm and head (llama.c:182-183)
     const int r = n - c0 < R ? n - c0 : R;
     rc |= qhip_rmsnorm_f32_rows(X + (size_t)c0 * dm, r, f->dm, f->g_final, f->eps, xn);
-    rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->head, f->vocab, lg, NULL);
+    rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->head, f->vocab, lg, NULL, pk);
     rc = rc || qhip_d2h_async(logits + (size_t)c0 * V, lg, (size_t)r * V * 4) || qhip_sync();
   }
   if (qhip_sync()) rc = 1;

@@ -80,6 +80,28 @@ def test_f32_gemv_group_edges_match_oracle(Q, K):
         ref.close()
 
 
+@pytest.mark.parametrize("rows,dff,vocab", [(1, 33, 70), (5, 64, 17), (9, 100, 130), (40, 31, 64), (70, 95, 2100),
+                                            (300, 66, 16384)])
+def test_f32_forward_tile_edges_match_oracle(Q, rows, dff, vocab):
+    """The many-row fp32 matmul where its tiles end: rows around a wave's and a
+    block's (each of the row groups of 1, 2, 4 and 8 is taken by one of these),
+    k rows past whole stages, batches and groups of four, column panels cut
+    short: every row bit for bit the oracle's step."""
+    cfg = [vocab, 144, 1, 3, 1, 48, dff, 320]
+    ref = O.FModel(cfg, 10000.0, seed=rows)
+    try:
+        g = gpu_model(Q, ref, cfg, 10000.0)
+        try:
+            ids = [(7 * i + 3) % vocab for i in range(rows)]
+            got = g.forward(ids)
+            for i, t in enumerate(ids):
+                assert np.array_equal(bits(got[i]), bits(ref.step(t))), (rows, i)
+        finally:
+            g.close()
+    finally:
+        ref.close()
+
+
 @pytest.mark.parametrize("shape", [(4096, 4096), (14336, 4096), (4096, 1024), (300, 17), (1000, 130), (129, 16)])
 def test_f32_gemv_rows_match_oracle(Q, shape):
     """The fp32 GEMV at (K, N) through a one-layer model whose down projection
