@@ -126,6 +126,137 @@ __device__ float seq_serial(int n, Term term) {
   return s;
 }
 
+// A thread's CM consecutive steps, classified.
+template <int CM>
+struct SeqSteps {
+  unsigned kp[CM];               // k total of the thread's steps before step c
+  int gh[CM];                    // grid after step c, were it hard
+  unsigned ks, hardmask;         // k total of the easy steps; bit c: step c is hard
+  int nh;                        // hard steps
+  int gin, gout;                 // grid of the first step if easy, else -1; grid of the run continuing past the last
+};
+
+// The terms a[] of one thread, whose partial sums are predicted to run from P0 to
+// P0 + loc within a relative rho; M0: bits of the largest term before them.  past:
+// the whole wave lies past the last term.  Wave-uniform control flow.
+template <int CM>
+__device__ __forceinline__ void seq_classify(const float (&a)[CM], float P0, float loc, unsigned M0, float rho,
+                                             bool past, SeqSteps<CM> &st) {
+  const float lo = 1.0f - rho, hi = 1.0f + rho;
+  unsigned ks = 0, hardmask = 0;
+  int nh = 0, gin = -1, gout = 0;
+  const int gA = seq_grid_max(P0 * lo, M0), gB = seq_grid((P0 + loc) * hi);
+  if (past) {
+    // a wave wholly past n holds only +0 terms, and s + 0 is s on any grid: no
+    // step to classify, no hard step, and no boundary to check (gin = -1)
+#pragma unroll
+    for (int c = 0; c < CM; c++) {
+      st.kp[c] = 0u;
+      st.gh[c] = 0;
+    }
+  } else if (__all(gA == gB)) {
+    // every chunk of the wave is predicted on one grid: only exact ties are hard
+    // (a term of the chunk is below the grid's binade top, so t < 2^24)
+#pragma unroll
+    for (int c = 0; c < CM; c++) {
+      const float t = ldexpf(a[c], 150 - gA);
+      const bool tie = __builtin_amdgcn_fractf(t) == 0.5f;
+      st.kp[c] = ks;
+      ks += tie ? 0u : (unsigned)__builtin_rintf(t);
+      nh += tie ? 1 : 0;
+      hardmask |= tie ? (1u << c) : 0u;
+      st.gh[c] = gA;
+    }
+    gin = (hardmask & 1u) ? -1 : gA;
+    gout = gA;
+  } else {
+    // (an easy step's term is below its grid's binade top, so t < 2^24; a hard
+    // step's t, possibly huge, is not used)
+    float P = P0;
+    unsigned L = M0;
+    int g0 = seq_grid_max(P * lo, L);
+#pragma unroll
+    for (int c = 0; c < CM; c++) {
+      const float Pn = P + a[c];
+      L = max(L, __float_as_uint(a[c]));
+      const int g1 = seq_grid(Pn * hi);
+      const float t = ldexpf(a[c], 150 - g0);
+      const bool easy = (g0 == g1) && (__builtin_amdgcn_fractf(t) != 0.5f);
+      st.kp[c] = ks;
+      ks += easy ? (unsigned)__builtin_rintf(t) : 0u;
+      nh += easy ? 0 : 1;
+      hardmask |= easy ? 0u : (1u << c);
+      if (c == 0) gin = easy ? g0 : -1;
+      const int gn = seq_grid_max(Pn * lo, L);           // the next step's grid: the grid after a hard step
+      st.gh[c] = gn;
+      gout = easy ? g0 : gn;                             // grid of the run continuing past this step
+      g0 = gn;
+      P = Pn;
+    }
+  }
+  st.ks = ks;
+  st.hardmask = hardmask;
+  st.nh = nh;
+  st.gin = gin;
+  st.gout = gout;
+}
+
+// One batch of the walk by one wave: lane i takes run m = base + i (the steps before
+// hard step m of htot; run htot is the tail) with the record cur of hard step m: k
+// total before it, index, term bits, grid after it.  (cx, cy, cw) carry the record
+// before the batch's first run from batch to batch, s the sum (lane 0).  Returns
+// whether every run of the batch is proven.
+template <typename Scratch>
+__device__ __forceinline__ bool seq_walk_batch(Scratch &S, const int4 &cur, int m, int base, int htot, float &s, int &cx,
+                                               int &cy, int &cw) {
+  const int lane = threadIdx.x & 63;
+  // the record before run m is lane m-1's (lane 0: the carry, DPP wave_shr:1)
+  const int px = __builtin_amdgcn_update_dpp(cx, cur.x, 0x138, 0xf, 0xf, false);
+  const int py = __builtin_amdgcn_update_dpp(cy, cur.y, 0x138, 0xf, 0xf, false);
+  const int gp = __builtin_amdgcn_update_dpp(cw, cur.w, 0x138, 0xf, 0xf, false);
+  cx = __builtin_amdgcn_readlane(cur.x, 63);
+  cy = __builtin_amdgcn_readlane(cur.y, 63);
+  cw = __builtin_amdgcn_readlane(cur.w, 63);
+  const unsigned K = (unsigned)cur.x - (unsigned)px;
+  const bool live = m <= htot && cur.y > py + 1;     // run m has steps
+  const float T = live ? ldexpf((float)K, gp - 150) : 0.0f;   // 0 past the tail: adds nothing
+  const float ah = __int_as_float(cur.z);                     // 0 from the tail on
+  // The serial part: lane 0 alone (exec holds one lane, so its LDS reads,
+  // adds and writes cost the least) adds the pairs in order, 8 at a time
+  // with the next 8 in flight, and records the partial sum each run starts
+  // from.  Pairs past the tail are (+0, +0) and leave s unchanged; the reads
+  // ahead past them stay inside walk[] and are not used.  A wave's LDS
+  // operations complete in order, so lane 0 reads what the wave has just
+  // written, and the wave reads back what lane 0 has written.
+  S.walk[lane] = make_float2(T, ah);
+  asm volatile("" ::: "memory");                      // keep the reads below the writes
+  if (lane == 0) {
+    const int cnt = min(64, htot + 1 - base);
+    const float4 *wp = reinterpret_cast<const float4 *>(S.walk);
+    float4 q0 = wp[0], q1 = wp[1], q2 = wp[2], q3 = wp[3];
+    for (int c = 0; c < cnt; c += 8) {
+      const float4 n0 = wp[(c >> 1) + 4], n1 = wp[(c >> 1) + 5], n2 = wp[(c >> 1) + 6], n3 = wp[(c >> 1) + 7];
+      float4 r0, r1;
+      r0.x = s; s = s + q0.x; s = s + q0.y;
+      r0.y = s; s = s + q0.z; s = s + q0.w;
+      r0.z = s; s = s + q1.x; s = s + q1.y;
+      r0.w = s; s = s + q1.z; s = s + q1.w;
+      r1.x = s; s = s + q2.x; s = s + q2.y;
+      r1.y = s; s = s + q2.z; s = s + q2.w;
+      r1.z = s; s = s + q3.x; s = s + q3.y;
+      r1.w = s; s = s + q3.z; s = s + q3.w;
+      *reinterpret_cast<float4 *>(&S.wst[c]) = r0;
+      *reinterpret_cast<float4 *>(&S.wst[c + 4]) = r1;
+      q0 = n0; q1 = n1; q2 = n2; q3 = n3;
+    }
+  }
+  asm volatile("" ::: "memory");
+  const float st = S.wst[lane];                       // read only where live
+  const float top = __uint_as_float((unsigned)(gp + 1) << 23);
+  const bool bad = live && !(K <= (1u << 23) && seq_grid(st) == gp && T <= top - st);
+  return !__any(bad);
+}
+
 // The sequential float32 sum of n terms, every one finite and >= 0.  Thread t
 // of the NT participating threads (threads 0 .. NT-1 of the block, NT a multiple
 // of 64, at most 1024) holds terms t*CM .. t*CM+CM-1 in a[], zero past n;
@@ -177,60 +308,10 @@ __device__ float seq_sum_nonneg(const float (&a)[CM], int n, SeqScratch &S, Term
   // error of the float scan that forms the prediction.  kp[c] is the k total of
   // this thread's steps before step c.
   const float rho = 0x1p-20f * __builtin_amdgcn_sqrtf((float)((tid + 1) * CM + 2)) + 0x1p-17f;
-  const float lo = 1.0f - rho, hi = 1.0f + rho;
-  unsigned ks = 0, hardmask = 0;
-  int nh = 0, gin = -1, gout = 0;
-  unsigned kp[CM];
-  int gh[CM];
-  const int gA = seq_grid_max(P0 * lo, M0), gB = seq_grid((P0 + loc) * hi);
-  if (wave * 64 * CM >= n) {
-    // a wave wholly past n holds only +0 terms, and s + 0 is s on any grid: no
-    // step to classify, no hard step, and no boundary to check (gin = -1)
-#pragma unroll
-    for (int c = 0; c < CM; c++) {
-      kp[c] = 0u;
-      gh[c] = 0;
-    }
-  } else if (__all(gA == gB)) {
-    // every chunk of the wave is predicted on one grid: only exact ties are hard
-    // (a term of the chunk is below the grid's binade top, so t < 2^24)
-#pragma unroll
-    for (int c = 0; c < CM; c++) {
-      const float t = ldexpf(a[c], 150 - gA);
-      const bool tie = __builtin_amdgcn_fractf(t) == 0.5f;
-      kp[c] = ks;
-      ks += tie ? 0u : (unsigned)__builtin_rintf(t);
-      nh += tie ? 1 : 0;
-      hardmask |= tie ? (1u << c) : 0u;
-      gh[c] = gA;
-    }
-    gin = (hardmask & 1u) ? -1 : gA;
-    gout = gA;
-  } else {
-    // (an easy step's term is below its grid's binade top, so t < 2^24; a hard
-    // step's t, possibly huge, is not used)
-    float P = P0;
-    unsigned L = M0;
-    int g0 = seq_grid_max(P * lo, L);
-#pragma unroll
-    for (int c = 0; c < CM; c++) {
-      const float Pn = P + a[c];
-      L = max(L, __float_as_uint(a[c]));
-      const int g1 = seq_grid(Pn * hi);
-      const float t = ldexpf(a[c], 150 - g0);
-      const bool easy = (g0 == g1) && (__builtin_amdgcn_fractf(t) != 0.5f);
-      kp[c] = ks;
-      ks += easy ? (unsigned)__builtin_rintf(t) : 0u;
-      nh += easy ? 0 : 1;
-      hardmask |= easy ? 0u : (1u << c);
-      if (c == 0) gin = easy ? g0 : -1;
-      const int gn = seq_grid_max(Pn * lo, L);           // the next step's grid: the grid after a hard step
-      gh[c] = gn;
-      gout = easy ? g0 : gn;                             // grid of the run continuing past this step
-      g0 = gn;
-      P = Pn;
-    }
-  }
+  SeqSteps<CM> st;
+  seq_classify<CM>(a, P0, loc, M0, rho, wave * 64 * CM >= n, st);
+  const unsigned ks = st.ks, hardmask = st.hardmask;
+  const int nh = st.nh, gin = st.gin, gout = st.gout;
 
   // 3. wave scans of the k totals and hard counts, the boundary check between
   // lanes, and the hard steps recorded in the wave's region in order (k totals
@@ -246,7 +327,7 @@ __device__ float seq_sum_nonneg(const float (&a)[CM], int n, SeqScratch &S, Term
 #pragma unroll
     for (int c = 0; c < CM; c++) {
       const bool h = (hardmask >> c) & 1u;
-      if (h) S.hs[m] = make_int4((int)(kb + kp[c]), tid * CM + c, __float_as_int(a[c]), gh[c]);
+      if (h) S.hs[m] = make_int4((int)(kb + st.kp[c]), tid * CM + c, __float_as_int(a[c]), st.gh[c]);
       m += h ? 1 : 0;
     }
   }
@@ -290,51 +371,7 @@ __device__ float seq_sum_nonneg(const float (&a)[CM], int n, SeqScratch &S, Term
         cur = S.hs[v * HCAP + m - hoff_v];
         cur.x = (int)((unsigned)cur.x + koff_v);
       }
-      // the record before run m is lane m-1's (lane 0: the carry, DPP wave_shr:1)
-      const int px = __builtin_amdgcn_update_dpp(cx, cur.x, 0x138, 0xf, 0xf, false);
-      const int py = __builtin_amdgcn_update_dpp(cy, cur.y, 0x138, 0xf, 0xf, false);
-      const int gp = __builtin_amdgcn_update_dpp(cw, cur.w, 0x138, 0xf, 0xf, false);
-      cx = __builtin_amdgcn_readlane(cur.x, 63);
-      cy = __builtin_amdgcn_readlane(cur.y, 63);
-      cw = __builtin_amdgcn_readlane(cur.w, 63);
-      const unsigned K = (unsigned)cur.x - (unsigned)px;
-      const bool live = m <= htot && cur.y > py + 1;     // run m has steps
-      const float T = live ? ldexpf((float)K, gp - 150) : 0.0f;   // 0 past the tail: adds nothing
-      const float ah = __int_as_float(cur.z);                     // 0 from the tail on
-      // The serial part: lane 0 alone (exec holds one lane, so its LDS reads,
-      // adds and writes cost the least) adds the pairs in order, 8 at a time
-      // with the next 8 in flight, and records the partial sum each run starts
-      // from.  Pairs past the tail are (+0, +0) and leave s unchanged; the reads
-      // ahead past them stay inside walk[] and are not used.  A wave's LDS
-      // operations complete in order, so lane 0 reads what the wave has just
-      // written, and the wave reads back what lane 0 has written.
-      S.walk[lane] = make_float2(T, ah);
-      asm volatile("" ::: "memory");                      // keep the reads below the writes
-      if (lane == 0) {
-        const int cnt = min(64, htot + 1 - base);
-        const float4 *wp = reinterpret_cast<const float4 *>(S.walk);
-        float4 q0 = wp[0], q1 = wp[1], q2 = wp[2], q3 = wp[3];
-        for (int c = 0; c < cnt; c += 8) {
-          const float4 n0 = wp[(c >> 1) + 4], n1 = wp[(c >> 1) + 5], n2 = wp[(c >> 1) + 6], n3 = wp[(c >> 1) + 7];
-          float4 r0, r1;
-          r0.x = s; s = s + q0.x; s = s + q0.y;
-          r0.y = s; s = s + q0.z; s = s + q0.w;
-          r0.z = s; s = s + q1.x; s = s + q1.y;
-          r0.w = s; s = s + q1.z; s = s + q1.w;
-          r1.x = s; s = s + q2.x; s = s + q2.y;
-          r1.y = s; s = s + q2.z; s = s + q2.w;
-          r1.z = s; s = s + q3.x; s = s + q3.y;
-          r1.w = s; s = s + q3.z; s = s + q3.w;
-          *reinterpret_cast<float4 *>(&S.wst[c]) = r0;
-          *reinterpret_cast<float4 *>(&S.wst[c + 4]) = r1;
-          q0 = n0; q1 = n1; q2 = n2; q3 = n3;
-        }
-      }
-      asm volatile("" ::: "memory");
-      const float st = S.wst[lane];                       // read only where live
-      const float top = __uint_as_float((unsigned)(gp + 1) << 23);
-      const bool bad = live && !(K <= (1u << 23) && seq_grid(st) == gp && T <= top - st);
-      ok = ok && !__any(bad);
+      ok = seq_walk_batch(S, cur, m, base, htot, s, cx, cy, cw) && ok;
     }
     if (!ok && lane == 0) s = seq_serial(n, term);
     if (lane == 0) {

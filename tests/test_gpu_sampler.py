@@ -57,6 +57,25 @@ def test_sample_token_paths_match_oracle(Q, V, k):
             assert t == r and rng.state == st, (V, k, kind)
 
 
+@pytest.mark.parametrize("V,k,p,kind", [
+    (1023, 40, 0.95, 0), (1024, 40, 1.0, 1), (4097, 64, 0.9, 0),          # fewer groups than k, one slice and its edges
+    (32000, 40, 0.95, 1), (70000, 1, 0.9, 0),                             # quarter-slice and slice maxima
+    (262144, 64, 1.0, 0), (262145, 64, 0.95, 0),                          # the split sum's widest vocabulary, and past it
+    (20000, 65, 0.9999, 0), (20000, 0, 1.0, 0), (20000, 0, 0.6, 1), (20000, 200, 1.0, 1)])   # kept lists over a wave
+def test_sample_token_split_sum_and_search_match_oracle(Q, V, k, p, kind):
+    """The sum over classified slices, the top-k bound from group maxima and the
+    search over the kept running sums, at the edges of each: tokens and rng states
+    of the oracle, over rows of several spreads and many equal logits (kind 1)."""
+    for tid, sigma, t in ((70, 0.3, 1.0), (71, 2.5, 0.8), (72, 8.0, 0.7)):
+        row = O.sample_row(V, tid, sigma, kind)
+        rng = Q.rng_create(tid)
+        st = O.rng_create(tid)
+        for _ in range(5):
+            g = Q.sample_token(row.reshape(1, -1), t, k, p, rng)
+            r, st = O.sample_token(row, t, k, p, st)
+            assert g == r and rng.state == st, (V, k, p, tid)
+
+
 def test_sample_argmax_first_index(Q):
     for tid in range(4):
         row = O.sample_row(128256 if tid % 2 else 32000, 30 + tid, 1.0, 1).reshape(1, -1)
