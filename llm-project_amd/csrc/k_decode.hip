@@ -210,9 +210,24 @@ __global__ void k_qacc_kn(const int8_t *qa, const int8_t *qw, int K, int N, int3
 }
 
 
+__global__ void k_stage_token(int *d_state, int *d_in, int pos, int token) {
+  if (threadIdx.x == 0) {
+    d_state[0] = pos;
+    d_state[1] = pos + 1;
+    d_in[pos] = token;
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+// One decode step's inputs (position state and token), as launch arguments: one
+// launch of a single wave instead of two copies of a few bytes from host memory.
+int qhip_stage_token(int *d_state, int *d_in, int pos, int token) {
+  QH_LAUNCH(QK_OTHER, k_stage_token, dim3(1), dim3(64), 0, d_state, d_in, pos, token);
+  return 0;
+}
 
 int qhip_embed(const int8_t *wte, const float *wte_s, int dm, const int *d_in, const int *d_state, float *x) {
   QH_LAUNCH(QK_EMBED, k_embed, dim3((dm + 255) / 256), dim3(256), 0, wte, wte_s, dm, d_in, d_state, x);

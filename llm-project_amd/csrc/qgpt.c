@@ -203,7 +203,7 @@ typedef struct {
   float *x, *xn, *qkv, *o, *h, *logits, *scores;
   int *d_state, *d_in;
   float *kbase, *vbase;                   // [L][nh][max_seq][hd]
-  int *h_stage;                           // pinned: position, end, token
+  float *h_logits;                        // pinned staging of the logits
   void *graph;
 } GDev;
 
@@ -212,7 +212,7 @@ static void gdev_free(GDev *g) {
   qhip_sync();
   if (g->graph) qhip_graph_destroy(g->graph);
   qhip_free(g->blob); qhip_free(g->kbase); qhip_free(g->vbase);
-  qhip_host_free(g->h_stage);
+  qhip_host_free(g->h_logits);
   free(g->wqkv); free(g->bqkv); free(g->wo); free(g->bo); free(g->g1); free(g->be1); free(g->g2); free(g->be2);
   free(g->w1); free(g->bf1); free(g->w2); free(g->bf2);
   free(g);
@@ -298,8 +298,8 @@ static GDev *gdev_create(const GPT *m) {
   const size_t per = (size_t)L * S * dm;                 // cache floats per K or V
   g->kbase = (float*)qhip_malloc(per * 4);
   g->vbase = (float*)qhip_malloc(per * 4);
-  g->h_stage = (int*)qhip_host_alloc(64);
-  if (!g->blob || !g->kbase || !g->vbase || !g->h_stage) {
+  g->h_logits = (float*)qhip_host_alloc((size_t)g->vocab * sizeof(float));
+  if (!g->blob || !g->kbase || !g->vbase || !g->h_logits) {
     fprintf(stderr, "Error: device allocation failed: %s\n", qhip_last_error());
     free(lo); gdev_free(g); return NULL;
   }
@@ -414,9 +414,7 @@ void gpt_decode_step(const GPT *m, KVCache *kv, int token, Tensor *logits) {
       abort();
     }
   }
-  int *h = g->h_stage;
-  h[0] = kv->len; h[1] = kv->len + 1; h[2] = token;
-  int rc = qhip_h2d_async(g->d_state, h, 2 * sizeof(int)) || qhip_h2d_async(g->d_in + kv->len, h + 2, sizeof(int));
+  int rc = qhip_stage_token(g->d_state, g->d_in, kv->len, token);
   if (!rc) {
     if (getenv("QLLAMA_NO_GRAPH") || qhip_profiling()) {
       rc = enqueue_gpt_step(g);
@@ -434,9 +432,10 @@ void gpt_decode_step(const GPT *m, KVCache *kv, int token, Tensor *logits) {
       if (!rc) rc = qhip_graph_launch(g->graph);
     }
   }
-  if (rc || qhip_d2h_async(logits->data, g->logits, (size_t)g->vocab * 4) || qhip_sync()) {
+  if (rc || qhip_d2h_async(g->h_logits, g->logits, (size_t)g->vocab * 4) || qhip_sync()) {
     fprintf(stderr, "Error: gpt_decode_step: %s\n", qhip_last_error());
     abort();
   }
+  memcpy(logits->data, g->h_logits, (size_t)g->vocab * 4);
   kv->len += 1;
 }

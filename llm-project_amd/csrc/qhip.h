@@ -35,6 +35,17 @@ int         qhip_flush_caches(void);                     // reads 512 MB: the ne
 int         qhip_upload_begin(size_t chunk);
 int         qhip_upload(void *dst, const void *host_src, size_t n);
 int         qhip_upload_end(void);
+// Staged download of results of the library stream to pageable host memory, beside
+// the launches enqueued after them: mark i (0 .. qhip_dl_max_marks() - 1) names
+// what has been enqueued when it is set, copy(i) takes n bytes that were ready
+// there, finish waits until every byte has reached the host.
+void *qhip_dl_create(size_t chunk);
+void qhip_dl_free(void *h);
+int qhip_dl_max_marks(void);
+void qhip_dl_prefault(void *dst, size_t n);   // bring the destination's pages in (host work, no device call)
+int qhip_dl_mark(void *h, int i);
+int qhip_dl_copy(void *h, int i, void *dst, const void *src, size_t n);
+int qhip_dl_finish(void *h);
 int         qhip_sync(void);
 void       *qhip_stream(void);
 
@@ -89,6 +100,7 @@ int qhip_hash_f32(const float *x, size_t n, uint64_t salt, uint64_t *out);
 
 // ---- decode kernels ------------------------------------------------------------
 // x[j] = (float)wte[token*dm + j] * s[j]   (llama.c:534-536), token = d_in[d_state[0]]
+int qhip_stage_token(int *d_state, int *d_in, int pos, int token);   // d_state = {pos, pos + 1}, d_in[pos] = token
 int qhip_embed(const int8_t *wte, const float *wte_s, int dm, const int *d_in, const int *d_state,
                float *x);
 // rows of x (rows, dm): y = rmsnorm(x) (rmsnorm.c:7-21), then per-row int8

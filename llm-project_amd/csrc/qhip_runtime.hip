@@ -1,10 +1,12 @@
 // qhip_runtime.hip - device, memory, stream, graph and event-timing services of the
 // HIP layer.  One stream per process carries every launch, in program order.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -176,9 +178,8 @@ struct Stager {
   int next = 0;
 } g_up;
 
-void par_copy(void *dst, const void *src, size_t n) {
-  const size_t kMinPart = (size_t)8 << 20;
-  const int parts = n >= 4 * kMinPart ? 4 : 1;
+void par_copy(void *dst, const void *src, size_t n, size_t min_part = (size_t)8 << 20) {
+  const int parts = n >= 4 * min_part ? 4 : 1;
   if (parts == 1) { memcpy(dst, src, n); return; }
   std::vector<std::thread> th;
   const size_t per = (n + parts - 1) / parts;
@@ -232,6 +233,111 @@ int qhip_upload_end(void) {
     g_up.busy[b] = false;
   }
   return rc;
+}
+
+// Staged download: device results of the library stream to pageable host memory
+// through two pinned buffers, on a copy stream of its own, so that the copies run
+// beside the launches that follow the results on the library stream; the CPU
+// empties one buffer while the other is filled.
+namespace {
+constexpr int kDlMarks = 16;
+struct Downloader {
+  hipStream_t stream = nullptr;
+  void *buf[2] = {nullptr, nullptr};
+  hipEvent_t ev[2] = {nullptr, nullptr}, mark[kDlMarks] = {};
+  void *dst[2] = {nullptr, nullptr};
+  size_t pend[2] = {0, 0}, chunk = 0;
+  int next = 0;            // the buffer to empty first
+};
+
+// Wait for buffer b's copy and hand its bytes to their host destination.
+int dl_empty(Downloader *d, int b) {
+  if (!d->pend[b]) return 0;
+  hipError_t e = hipEventSynchronize(d->ev[b]);
+  if (e != hipSuccess) return fail("download wait", e);
+  par_copy(d->dst[b], d->buf[b], d->pend[b], (size_t)2 << 20);
+  d->pend[b] = 0;
+  return 0;
+}
+}  // namespace
+
+void qhip_dl_free(void *h) {
+  Downloader *d = static_cast<Downloader *>(h);
+  if (!d) return;
+  if (d->stream) (void)hipStreamSynchronize(d->stream);
+  for (int b = 0; b < 2; b++) {
+    if (d->buf[b]) (void)hipHostFree(d->buf[b]);
+    if (d->ev[b]) (void)hipEventDestroy(d->ev[b]);
+  }
+  for (int i = 0; i < kDlMarks; i++)
+    if (d->mark[i]) (void)hipEventDestroy(d->mark[i]);
+  if (d->stream) (void)hipStreamDestroy(d->stream);
+  delete d;
+}
+
+void *qhip_dl_create(size_t chunk) {
+  Downloader *d = new (std::nothrow) Downloader();
+  if (!d) return nullptr;
+  d->chunk = chunk;
+  hipError_t e = hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking);
+  for (int b = 0; b < 2 && e == hipSuccess; b++) {
+    e = hipHostMalloc(&d->buf[b], chunk, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&d->ev[b], hipEventDisableTiming);
+  }
+  for (int i = 0; i < kDlMarks && e == hipSuccess; i++) e = hipEventCreateWithFlags(&d->mark[i], hipEventDisableTiming);
+  if (e != hipSuccess) {
+    fail("download staging", e);
+    (void)hipGetLastError();
+    qhip_dl_free(d);
+    return nullptr;
+  }
+  return d;
+}
+
+// Have the pages of a destination present before its copies: where they were never
+// written, the CPU's copies would otherwise take a fault each.  The bytes stay as
+// they are; a kernel that does not know the request refuses it, and the faults stay.
+void qhip_dl_prefault(void *dst, size_t n) {
+#ifdef MADV_POPULATE_WRITE
+  const uintptr_t page = 4096, a = ((uintptr_t)dst + page - 1) & ~(page - 1), e = ((uintptr_t)dst + n) & ~(page - 1);
+  if (e > a + ((uintptr_t)1 << 20)) (void)madvise((void *)a, e - a, MADV_POPULATE_WRITE);
+#else
+  (void)dst; (void)n;
+#endif
+}
+
+int qhip_dl_max_marks(void) { return kDlMarks; }
+
+// Mark the results enqueued so far on the library stream (i = 0 .. kDlMarks - 1).
+int qhip_dl_mark(void *h, int i) {
+  hipError_t e = hipEventRecord(static_cast<Downloader *>(h)->mark[i], g_stream);
+  return e == hipSuccess ? 0 : fail("download mark", e);
+}
+
+// Copy n bytes that were ready at mark i; the last two chunks are in flight or in
+// the buffers on return.
+int qhip_dl_copy(void *h, int i, void *dst, const void *src, size_t n) {
+  Downloader *d = static_cast<Downloader *>(h);
+  hipError_t e = hipStreamWaitEvent(d->stream, d->mark[i], 0);
+  if (e != hipSuccess) return fail("download order", e);
+  for (size_t o = 0; o < n; o += d->chunk) {
+    const size_t c = n - o < d->chunk ? n - o : d->chunk;
+    const int b = d->next;       // the buffer whose copy was enqueued first
+    if (dl_empty(d, b)) return 1;
+    if ((e = hipMemcpyAsync(d->buf[b], (const char *)src + o, c, hipMemcpyDeviceToHost, d->stream)) != hipSuccess ||
+        (e = hipEventRecord(d->ev[b], d->stream)) != hipSuccess)
+      return fail("download copy", e);
+    d->dst[b] = (char *)dst + o;
+    d->pend[b] = c;
+    d->next = b ^ 1;
+  }
+  return 0;
+}
+
+int qhip_dl_finish(void *h) {
+  Downloader *d = static_cast<Downloader *>(h);
+  const int b = d->next;
+  return dl_empty(d, b) | dl_empty(d, b ^ 1);
 }
 
 int qhip_copy2d_d2d(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t height) {

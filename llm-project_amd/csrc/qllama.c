@@ -764,6 +764,7 @@ static int run_steps(const QDev *d, KVDev *kd, int n) {
 
 // Stage tokens ids[0..n) at positions pos..pos+n-1 and set (pos, fill_end).
 static int stage_inputs(const QDev *d, int pos, const int *ids, int n) {
+  if (n == 1) return qhip_stage_token(d->d_state, d->d_in, pos, ids[0]);
   int *h = d->h_stage;
   h[0] = pos; h[1] = pos + n;
   if (qhip_h2d_async(d->d_state, h, 2 * sizeof(int))) return 1;
@@ -951,25 +952,38 @@ typedef struct FDev {
   float *wte, *head, *g_final, *rope_cos, *rope_sin;
   float *x, *xn, *qkv, *o, *gu, *h, *logits, *scores;
   int *d_state, *d_in;
-  int *h_stage;
+  float *h_logits;     // pinned staging of one row of logits
+  void *ws;            // the batched forward's workspace, grown to the longest call
+  size_t ws_bytes;
 } FDev;
 
 #define FDEV_MAX 16
 static FDev *g_fdev[FDEV_MAX];
+// The pinned staging the batched forward's logits come back through: one for the
+// process (two chunks of FWD_DL_CHUNK), made by the first forward and given back
+// with the last fp32 model.
+#define FWD_DL_CHUNK ((size_t)8 << 20)
+static void *g_fwd_dl;
 
 static void fdev_free(FDev *f) {
   if (!f) return;
   qhip_free(f->blob);
-  qhip_host_free(f->h_stage);
+  qhip_host_free(f->h_logits);
+  qhip_free(f->ws);
   free(f->wqkv); free(f->bqkv); free(f->wo); free(f->wgu); free(f->wd); free(f->g_attn); free(f->g_ffn);
   free(f);
 }
 
 static void fdev_release(FDev *f) {
   if (--f->refs > 0) return;
-  for (int i = 0; i < FDEV_MAX; i++) if (g_fdev[i] == f) g_fdev[i] = NULL;
+  int others = 0;
+  for (int i = 0; i < FDEV_MAX; i++) {
+    if (g_fdev[i] == f) g_fdev[i] = NULL;
+    if (g_fdev[i]) others = 1;
+  }
   qhip_sync();
   fdev_free(f);
+  if (!others) { qhip_dl_free(g_fwd_dl); g_fwd_dl = NULL; }
 }
 
 static FDev *fdev_find(const LlamaModel *m) {
@@ -1026,11 +1040,11 @@ static FDev *fdev_upload(const LlamaModel *m) {
   if (dm * nqkv > big) big = dm * nqkv;
   if (qd * dm > big) big = qd * dm;
   f->blob = (uint8_t*)qhip_malloc(off);
-  f->h_stage = (int*)qhip_host_alloc(64);
+  f->h_logits = (float*)qhip_host_alloc(V * sizeof(float));
   float *tmp = (float*)qhip_malloc(big * 4);
   size_t big2 = dm * (qd > dff ? qd : dff);                // one part of a joined matrix
   float *tmp2 = (float*)qhip_malloc(big2 * 4);
-  if (!f->blob || !f->h_stage || !tmp || !tmp2) {
+  if (!f->blob || !f->h_logits || !tmp || !tmp2) {
     fprintf(stderr, "Error: device allocation of %zu bytes failed: %s\n", off, qhip_last_error());
     qhip_free(tmp); qhip_free(tmp2); free(lo); fdev_free(f); return NULL;
   }
@@ -1137,9 +1151,7 @@ void llama_decode_step(const LlamaModel *m, LlamaKV *kv, int token, Tensor *logi
     fprintf(stderr, "Error: llama_decode_step: position %d / token %d out of range\n", kv->len, token);
     abort();
   }
-  int *h = f->h_stage;
-  h[0] = kv->len; h[1] = kv->len + 1; h[2] = token;
-  int rc = qhip_h2d_async(f->d_state, h, 2 * sizeof(int)) || qhip_h2d_async(f->d_in + kv->len, h + 2, sizeof(int));
+  int rc = qhip_stage_token(f->d_state, f->d_in, kv->len, token);
   if (!rc) {
     if (profiling || getenv("QLLAMA_NO_GRAPH")) {
       rc = enqueue_step_f32(f, kd);
@@ -1158,7 +1170,8 @@ void llama_decode_step(const LlamaModel *m, LlamaKV *kv, int token, Tensor *logi
       if (!rc) rc = qhip_graph_launch(kd->graph);
     }
   }
-  if (rc || qhip_d2h_async(logits->data, f->logits, (size_t)f->vocab * 4) || qhip_sync()) die("llama_decode_step");
+  if (rc || qhip_d2h_async(f->h_logits, f->logits, (size_t)f->vocab * 4) || qhip_sync()) die("llama_decode_step");
+  memcpy(logits->data, f->h_logits, (size_t)f->vocab * 4);
   kv->len += 1;
 }
 
@@ -1184,7 +1197,7 @@ static int fwd_supported(const FDev *f) {
   return (f->hd == 128 || f->hd == 64 || f->hd == 48) && G >= 1 && G <= 8 && G * f->hd <= 1024;
 }
 
-static int fwd_run(const FDev *f, float rope_base, const int *ids, int n, float *logits) {
+static int fwd_run(FDev *f, float rope_base, const int *ids, int n, float *logits) {
   const int R = n < FWD_ROWS ? n : FWD_ROWS, half = f->hd / 2, own_rope = n > f->max_seq;
   const size_t dm = (size_t)f->dm, V = (size_t)f->vocab, per = (size_t)f->KVH * n * f->hd;
   size_t off = 0;
@@ -1198,8 +1211,15 @@ static int fwd_run(const FDev *f, float rope_base, const int *ids, int n, float 
   if (f->dff > kmax) kmax = f->dff;
   const size_t o_pk = FTAKE(qhip_gemm_f32_pack(R, kmax));
 #undef FTAKE
-  uint8_t *b = (uint8_t*)qhip_malloc(off);
-  if (!b) return 1;
+  if (f->ws_bytes < off) {
+    qhip_sync();
+    qhip_free(f->ws);
+    f->ws = qhip_malloc(off);
+    f->ws_bytes = f->ws ? off : 0;
+  }
+  if (!g_fwd_dl) g_fwd_dl = qhip_dl_create(FWD_DL_CHUNK);
+  uint8_t *b = (uint8_t*)f->ws;
+  if (!b || !g_fwd_dl) return 1;
   int *d_ids = (int*)(b + o_ids);
   float *X = (float*)(b + o_x), *xn = (float*)(b + o_xn), *qkv = (float*)(b + o_qkv), *q = (float*)(b + o_q);
   float *o = (float*)(b + o_o), *gu = (float*)(b + o_gu), *h = (float*)(b + o_h), *lg = (float*)(b + o_lg);
@@ -1225,14 +1245,29 @@ static int fwd_run(const FDev *f, float rope_base, const int *ids, int n, float 
       rc |= qhip_swiglu_f32_rows(gu, r, f->dff, h);
       rc |= qhip_gemm_f32(1, FWD_CLS, h, r, f->dff, f->wd[l], f->dm, Xc, NULL, pk);
     }
-  for (int c0 = 0; c0 < n && !rc; c0 += R) {   // final norm and head (llama.c:182-183)
+  // final norm and head (llama.c:182-183), in parts of whole 64-row tiles with about
+  // a staged copy of logits each: a part's logits go to the host while the next
+  // parts are computed
+  const int most = qhip_dl_max_marks();
+  for (int c0 = 0; c0 < n && !rc; c0 += R) {
     const int r = n - c0 < R ? n - c0 : R;
+    int part = (int)(FWD_DL_CHUNK / (V * 4)) / 64 * 64;
+    if (part < 64) part = 64;
+    if ((r + part - 1) / part > most) part = ((r + most - 1) / most + 63) / 64 * 64;
     rc |= qhip_rmsnorm_f32_rows(X + (size_t)c0 * dm, r, f->dm, f->g_final, f->eps, xn);
-    rc |= qhip_gemm_f32(0, FWD_CLS, xn, r, f->dm, f->head, f->vocab, lg, NULL, pk);
-    rc = rc || qhip_d2h_async(logits + (size_t)c0 * V, lg, (size_t)r * V * 4) || qhip_sync();
+    for (int p0 = 0, i = 0; p0 < r && !rc; p0 += part, i++) {
+      const int pr = r - p0 < part ? r - p0 : part;
+      rc |= qhip_gemm_f32(0, FWD_CLS, xn + (size_t)p0 * dm, pr, f->dm, f->head, f->vocab, lg + p0 * V, NULL, pk);
+      rc = rc || qhip_dl_mark(g_fwd_dl, i);
+    }
+    if (!rc) qhip_dl_prefault(logits + (size_t)c0 * V, (size_t)r * V * 4);    // while the GPU is at the layers
+    for (int p0 = 0, i = 0; p0 < r && !rc; p0 += part, i++) {
+      const int pr = r - p0 < part ? r - p0 : part;
+      rc = qhip_dl_copy(g_fwd_dl, i, logits + ((size_t)c0 + p0) * V, lg + p0 * V, (size_t)pr * V * 4);
+    }
+    if (qhip_dl_finish(g_fwd_dl)) rc = 1;
   }
   if (qhip_sync()) rc = 1;
-  qhip_free(b);
   return rc;
 }
 
