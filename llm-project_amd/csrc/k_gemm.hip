@@ -11,12 +11,14 @@
 //   SWIGLU gate j and up j -> h = (g * (1 / (1 + expf(-g)))) * u  (llama.c:583-587)
 //
 // Operands are K-contiguous (activation rows [M][kpad], weight rows [N][kpad]).
-// Two kernels, both in K steps of 64 bytes through LDS:
-//  - k_gemm_i8_pipe (kpad % 64 == 0): block tiles of 128 x 128 or 256 x 128 (SWIGLU:
-//    half the columns are gate rows, half the matching up rows), 8 waves of
-//    v_mfma_i32_32x32x32_i8 (the 16x16x64 form runs at half its rate on gfx950).
-//    Both operand tiles are copied straight from global memory into LDS
-//    (global_load_lds, no staging registers), three or four K steps ahead.
+// Three kernels (launch() chooses):
+//  - k_gemm_i8_deep (kpad % 128 == 0): block tiles of 256 x 256, 256 x 128 or 128 x 128
+//    (SWIGLU: half the columns are gate rows, half the matching up rows) in K steps
+//    of 128 bytes, v_mfma_i32_32x32x32_i8 (the 16x16x64 form runs at half its rate on
+//    gfx950).  Both operand tiles are copied straight from global memory into LDS
+//    (global_load_lds, no staging registers), two to four K steps in LDS.
+//  - k_gemm_i8_pipe (kpad % 64 == 0): 128 x 128 tiles, K steps of 64 bytes, 8 waves,
+//    four steps in LDS.
 //  - k_gemm_i8 (other K): 128 x 128 tiles staged through registers into
 //    double-buffered LDS, 4 waves of 4 x 4 v_mfma_i32_16x16x64_i8; chunks past
 //    kpad are zero.
@@ -212,6 +214,137 @@ __device__ __forceinline__ void block_sync_lds() {
   asm volatile("" ::: "memory");
 }
 
+// What a block's epilogue reads besides the sums, requested before its K loop: the
+// scales of its TM rows and (SwiGLU) the exp table in LDS, and a lane's column
+// scales and biases in registers.  (Read element by element between the stores,
+// which the compiler has to keep in order, they cost a memory round trip each: 28 of
+// 82 us of the QKV product at 2048 rows, 91 of 300 of gate|up.)
+template <int TM>
+struct EpiShared {
+  __attribute__((aligned(16))) float as[TM];
+  uint64_t tab[32];
+};
+
+template <int MODE>
+struct EpiLane {
+  int j[2];            // output columns of the two column blocks (SwiGLU: one, its gate and up scales in w)
+  float w[2], b[2];
+};
+
+// All threads; published by the first barrier of the K loop.
+template <int MODE, int TM, int NT>
+__device__ __forceinline__ EpiLane<MODE> epi_begin(EpiShared<TM> &sh, const float *as, const float *ws,
+                                                   const float *bias, int M, int N, int m0, int n0, int wn, int lane) {
+  for (int r = threadIdx.x; r < TM; r += NT) sh.as[r] = as[min(m0 + r, M - 1)];
+  if (MODE == GM_SWIGLU && threadIdx.x < 32) sh.tab[threadIdx.x] = qd::kExp2Tab[threadIdx.x];
+  EpiLane<MODE> l;
+  if (MODE == GM_SWIGLU) {
+    l.j[0] = l.j[1] = n0 + wn * 32 + (lane & 31);
+    l.w[0] = ws[min(l.j[0], N - 1)];
+    l.w[1] = ws[N + min(l.j[0], N - 1)];
+    l.b[0] = l.b[1] = 0.0f;
+  } else {
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      l.j[b] = n0 + wn * 64 + b * 32 + (lane & 31);
+      l.w[b] = ws[min(l.j[b], N - 1)];
+      l.b[b] = MODE == GM_PLAIN && bias ? bias[min(l.j[b], N - 1)] : 0.0f;
+    }
+  }
+  return l;
+}
+
+// The wave's sums to the output: result element e of row block a is row i0 + 32 a +
+// 8 (e / 4) + 4 (lane / 32) + e % 4, i0 = r0 rows into the block's m0.  FULL: every
+// row and column of the block exists.  The decode GEMV's operations and order.
+template <int MODE, int RB, int TM, bool FULL>
+__device__ __forceinline__ void epi_store(const v16i (&acc)[RB][2], const EpiShared<TM> &sh, const EpiLane<MODE> &l,
+                                          bool has_bias, int M, int N, float *__restrict__ out, int ldo, int m0,
+                                          int r0, int lane) {
+  const int rl = r0 + 4 * (lane >> 5);
+  auto row = [&](int a, int e) { return 32 * a + 8 * (e >> 2) + (e & 3); };      // from row m0 + rl
+  float *o0 = out + (size_t)(m0 + rl) * ldo + l.j[0];
+  const int step = l.j[1] - l.j[0];                                              // 32 (SwiGLU: 0)
+  float old[2][MODE == GM_RESID ? 16 : 1][2];
+  auto fetch = [&](int a) __attribute__((always_inline)) {
+    if constexpr (MODE == GM_RESID) {
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+          old[a & 1][e][b] = FULL || (m0 + rl + row(a, e) < M && l.j[b] < N) ? o0[(size_t)row(a, e) * ldo + b * step] : 0.0f;
+    }
+  };
+  fetch(0);
+#pragma unroll
+  for (int a = 0; a < RB; a++) {
+    if (a + 1 < RB) fetch(a + 1);                    // requested before this block's stores
+    float s[16];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const float4 t = *reinterpret_cast<const float4 *>(&sh.as[rl + 32 * a + 8 * q]);
+      s[4 * q] = t.x; s[4 * q + 1] = t.y; s[4 * q + 2] = t.z; s[4 * q + 3] = t.w;
+    }
+    if constexpr (MODE == GM_SWIGLU) {
+#pragma unroll
+      for (int h = 0; h < 16; h += 8) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = -((s[h + e] * l.w[0]) * (float)acc[a][0][h + e]);
+        float g[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) g[e] = -x[e];
+        qd::expf_glibc_n<8>(x, sh.tab);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float up = (s[h + e] * l.w[1]) * (float)acc[a][1][h + e];
+          const float sg = 1.0f / (1.0f + x[e]);
+          if (FULL || (m0 + rl + row(a, h + e) < M && l.j[0] < N)) o0[(size_t)row(a, h + e) * ldo] = (g[e] * sg) * up;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+          const float c = (s[e] * l.w[b]) * (float)acc[a][b][e];
+          float v;
+          if constexpr (MODE == GM_RESID) v = old[a & 1][e][b] + c;
+          else v = has_bias ? c + l.b[b] : c;
+          if (FULL || (m0 + rl + row(a, e) < M && l.j[b] < N)) o0[(size_t)row(a, e) * ldo + b * step] = v;
+        }
+    }
+  }
+}
+
+// int32 partial sums of K split `split` to part[split][M][N] (SwiGLU: [split][M][2N], up
+// columns at N + j).
+template <int MODE, int RB>
+__device__ __forceinline__ void epi_part(const v16i (&acc)[RB][2], const EpiLane<MODE> &l, int M, int N, int *part,
+                                         int split, int i0, int lane) {
+  const int ldp = MODE == GM_SWIGLU ? 2 * N : N;
+  int *pp = part + (size_t)split * M * ldp;
+#pragma unroll
+  for (int a = 0; a < RB; a++) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int i = i0 + a * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+      if (i >= M) continue;
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+        if (l.j[b] < N) pp[(size_t)i * ldp + (MODE == GM_SWIGLU && b ? N : 0) + l.j[b]] = acc[a][b][e];
+    }
+  }
+}
+
+template <int MODE, int RB, int TM>
+__device__ __forceinline__ void epi_end(const v16i (&acc)[RB][2], const EpiShared<TM> &sh, const EpiLane<MODE> &l,
+                                        bool has_bias, int M, int N, float *out, int ldo, int m0, int n0, int nout,
+                                        int r0, int lane) {
+  if (m0 + TM <= M && n0 + nout <= N) epi_store<MODE, RB, TM, true>(acc, sh, l, has_bias, M, N, out, ldo, m0, r0, lane);
+  else epi_store<MODE, RB, TM, false>(acc, sh, l, has_bias, M, N, out, ldo, m0, r0, lane);
+}
+
 // Block tile TM x TN, waves WM x WN, each wave (TM/WM) x (TN/WN) from 32 x 32
 // v_mfma_i32_32x32x32_i8 blocks: RB row blocks x 2 column blocks (SWIGLU: the
 // wave's 32 gate columns and the matching 32 up columns).
@@ -246,6 +379,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_i8_pipe(const int8_t *A, 
   const int m0 = mtile * TM;
   constexpr int NOUT = MODE == GM_SWIGLU ? TN / 2 : TN;
   const int n0 = ntile * NOUT;
+  __shared__ EpiShared<TM> epi;
+  const EpiLane<MODE> el = epi_begin<MODE, TM, 64 * NWAVE>(epi, as, ws, bias, M, N, m0, n0, wn, lane);
 
   // this lane's global chunks: wave instructions wave*LA + i of the A tile and
   // wave*LB + i of the B tile
@@ -361,63 +496,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_i8_pipe(const int8_t *A, 
     if (NSTAGE > 3 && kt + 3 < nk) step(std::integral_constant<int, (NSTAGE > 3 ? 3 : 0)>(), kt + 3);
   }
 
-  if constexpr (PART) {                // int32 partial sums of this split
-    const int ldp = MODE == GM_SWIGLU ? 2 * N : N;
-    int *pp = part + (size_t)split * M * ldp;
-#pragma unroll
-    for (int a = 0; a < RB; a++) {
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int i = m0 + wm * (TM / WM) + a * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-        if (i >= M) continue;
-        if (MODE == GM_SWIGLU) {
-          const int j = n0 + wn * 32 + (lane & 31);
-          if (j < N) {
-            pp[(size_t)i * ldp + j] = acc[a][0][e];
-            pp[(size_t)i * ldp + N + j] = acc[a][1][e];
-          }
-        } else {
-#pragma unroll
-          for (int b = 0; b < 2; b++) {
-            const int j = n0 + wn * 64 + b * 32 + (lane & 31);
-            if (j < N) pp[(size_t)i * ldp + j] = acc[a][b][e];
-          }
-        }
-      }
-    }
-    return;
-  }
-
-  // epilogue (the decode GEMV's operations and order)
-#pragma unroll
-  for (int a = 0; a < RB; a++) {
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const int i = m0 + wm * (TM / WM) + a * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      if (i >= M) continue;
-      const float asi = as[i];
-      if (MODE == GM_SWIGLU) {
-        const int j = n0 + wn * 32 + (lane & 31);
-        if (j < N) {
-          const float g = (asi * ws[j]) * (float)acc[a][0][e];
-          const float up = (asi * ws[N + j]) * (float)acc[a][1][e];
-          const float s = 1.0f / (1.0f + qd::expf_glibc(-g));
-          out[(size_t)i * ldo + j] = (g * s) * up;
-        }
-      } else {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-          const int j = n0 + wn * 64 + b * 32 + (lane & 31);
-          if (j < N) {
-            const float c = (asi * ws[j]) * (float)acc[a][b][e];
-            float *o = out + (size_t)i * ldo + j;
-            if (MODE == GM_RESID) *o = *o + c;
-            else *o = bias ? c + bias[j] : c;
-          }
-        }
-      }
-    }
-  }
+  if constexpr (PART) epi_part<MODE, RB>(acc, el, M, N, part, split, m0 + wm * (TM / WM), lane);
+  else epi_end<MODE, RB, TM>(acc, epi, el, bias != nullptr, M, N, out, ldo, m0, n0, NOUT, wm * (TM / WM), lane);
 }
 
 constexpr int kMaxSplits = 16;         // K splits of one GEMM at most
@@ -497,19 +577,245 @@ int launch_pipe(const int8_t *A, const float *as, const int8_t *W, const float *
   return 0;
 }
 
-// Tile choice (measured at the 8B prefill shapes, M = 2048): 256 x 128 blocks for
-// the wide gate|up GEMM and for long K; 128 x 128 blocks of 8 waves otherwise.
-// K not a multiple of 64 takes the register-staged kernel.
+// ---------------------------------------------------------------------------
+// Deep variant for kpad % 128 == 0 and many rows: K steps of 128 bytes, so that a
+// copy instruction moves eight whole 128-byte lines (64-byte rows cost the cache a
+// line each for half its bytes), and a loop whose LDS reads, copies and products
+// overlap by construction.  Staged rows are 128 bytes, 16-byte chunk c of row r at
+// slot c ^ ((r >> 1) & 7): 16 consecutive rows read at one c fall in distinct banks.
+//
+// A step is four phases of 32 K bytes.  A phase reads the next phase's fragments
+// while it multiplies its own (2 * RB products) and ends when they have arrived:
+// one asm block, so that no register holds a load in flight outside it.  The one
+// barrier of a step sits before its last phase: every wave has then read all of the
+// step's fragments, so its buffer takes the copies of step + NS, and the copies of
+// the next step, issued NS - 1 steps ago, have landed for the reads of that phase.
+// ---------------------------------------------------------------------------
+constexpr int DK = 128;
+
+__device__ __forceinline__ int swz_deep(int r) { return (r >> 1) & 7; }
+
+#define DP_RD(dst, base, off) "ds_read_b128 %[" dst "], %[" base "] offset:" off "\n\t"
+#define DP_MM(c, a, b) "v_mfma_i32_32x32x32_i8 %[" c "], %[" a "], %[" b "], %[" c "]\n\t"
+
+// acc += fragments (fa, fb); (na, nb) = the fragments at LDS addresses la, lb (row
+// blocks 4096 bytes apart, the second column block BOFF bytes on).
+template <int BOFF>
+__device__ __forceinline__ void gemm_phase(v16i (&acc)[4][2], const v4i (&fa)[4], const v4i (&fb)[2], v4i (&na)[4],
+                                           v4i (&nb)[2], unsigned la, unsigned lb) {
+  asm volatile(
+      DP_RD("nb0", "lb", "0") DP_RD("na0", "la", "0") DP_MM("c00", "a0", "b0")
+      DP_RD("nb1", "lb", "%[bo]") DP_MM("c01", "a0", "b1")
+      DP_RD("na1", "la", "4096") DP_MM("c10", "a1", "b0")
+      DP_RD("na2", "la", "8192") DP_MM("c11", "a1", "b1")
+      DP_RD("na3", "la", "12288") DP_MM("c20", "a2", "b0")
+      DP_MM("c21", "a2", "b1") DP_MM("c30", "a3", "b0") DP_MM("c31", "a3", "b1")
+      "s_waitcnt lgkmcnt(0)"
+      : [c00] "+v"(acc[0][0]), [c01] "+v"(acc[0][1]), [c10] "+v"(acc[1][0]), [c11] "+v"(acc[1][1]),
+        [c20] "+v"(acc[2][0]), [c21] "+v"(acc[2][1]), [c30] "+v"(acc[3][0]), [c31] "+v"(acc[3][1]),
+        [na0] "=&v"(na[0]), [na1] "=&v"(na[1]), [na2] "=&v"(na[2]), [na3] "=&v"(na[3]), [nb0] "=&v"(nb[0]),
+        [nb1] "=&v"(nb[1])
+      : [a0] "v"(fa[0]), [a1] "v"(fa[1]), [a2] "v"(fa[2]), [a3] "v"(fa[3]), [b0] "v"(fb[0]), [b1] "v"(fb[1]),
+        [la] "v"(la), [lb] "v"(lb), [bo] "n"(BOFF)
+      : "memory");
+}
+
+template <int BOFF>
+__device__ __forceinline__ void gemm_phase(v16i (&acc)[2][2], const v4i (&fa)[2], const v4i (&fb)[2], v4i (&na)[2],
+                                           v4i (&nb)[2], unsigned la, unsigned lb) {
+  asm volatile(
+      DP_RD("nb0", "lb", "0") DP_RD("na0", "la", "0") DP_MM("c00", "a0", "b0")
+      DP_RD("nb1", "lb", "%[bo]") DP_MM("c01", "a0", "b1")
+      DP_RD("na1", "la", "4096") DP_MM("c10", "a1", "b0")
+      DP_MM("c11", "a1", "b1")
+      "s_waitcnt lgkmcnt(0)"
+      : [c00] "+v"(acc[0][0]), [c01] "+v"(acc[0][1]), [c10] "+v"(acc[1][0]), [c11] "+v"(acc[1][1]),
+        [na0] "=&v"(na[0]), [na1] "=&v"(na[1]), [nb0] "=&v"(nb[0]), [nb1] "=&v"(nb[1])
+      : [a0] "v"(fa[0]), [a1] "v"(fa[1]), [b0] "v"(fb[0]), [b1] "v"(fb[1]), [la] "v"(la), [lb] "v"(lb), [bo] "n"(BOFF)
+      : "memory");
+}
+#undef DP_RD
+#undef DP_MM
+
+template <int MODE, int TM, int TN, int WM, int WN, int NS, bool PART = false>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_i8_deep(
+    const int8_t *A, const float *as, const int8_t *W, const float *ws, int M, int N, int kpad, float *out, int ldo,
+    const float *bias, int mt_count, int nt_count, int bps, int nks, int *part) {
+  constexpr int NWAVE = WM * WN, RB = TM / WM / 32;
+  static_assert(TN == 64 * WN, "two 32-column blocks per wave");
+  static_assert(TM % (8 * NWAVE) == 0 && TN % (8 * NWAVE) == 0, "whole wave instructions per tile");
+  constexpr int LA = TM / 8 / NWAVE, LB = TN / 8 / NWAVE, LPS = LA + LB;     // 1 KiB copies per wave and step
+  constexpr int STAGE = (TM + TN) * DK;
+  constexpr int BOFF = (MODE == GM_SWIGLU ? TN / 2 : 32) * DK;
+  __shared__ __attribute__((aligned(1024))) int8_t lds[NS * STAGE];
+  int mtile, ntile;
+  const int split = PART ? (int)blockIdx.x / bps : 0;              // as in k_gemm_i8_pipe
+  gemm_tile(PART ? (int)blockIdx.x % bps : (int)blockIdx.x, mt_count, mtile, ntile);
+  if (ntile >= nt_count) return;                                   // uniform for the block
+  const int kt0 = split * nks;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int m0 = mtile * TM;
+  constexpr int NOUT = MODE == GM_SWIGLU ? TN / 2 : TN;
+  const int n0 = ntile * NOUT;
+  __shared__ EpiShared<TM> epi;
+  const EpiLane<MODE> el = epi_begin<MODE, TM, 64 * NWAVE>(epi, as, ws, bias, M, N, m0, n0, wn, lane);
+
+  // this lane's bytes of copy instruction i of each operand: row 8 * (wave * L + i) + lane / 8 of the
+  // tile, the chunk that the swizzle puts at slot lane % 8
+  const int8_t *ga[LA], *gb[LB];
+#pragma unroll
+  for (int i = 0; i < LA; i++) {
+    const int row = 8 * (wave * LA + i) + (lane >> 3), c = (lane & 7) ^ swz_deep(row);
+    ga[i] = A + (size_t)min(m0 + row, M - 1) * kpad + c * 16 + (size_t)kt0 * DK;
+  }
+#pragma unroll
+  for (int i = 0; i < LB; i++) {
+    const int row = 8 * (wave * LB + i) + (lane >> 3), c = (lane & 7) ^ swz_deep(row);
+    int wrow;
+    if (MODE == GM_SWIGLU) wrow = row < TN / 2 ? min(n0 + row, N - 1) : N + min(n0 + row - TN / 2, N - 1);
+    else wrow = min(n0 + row, N - 1);
+    gb[i] = W + (size_t)wrow * kpad + c * 16 + (size_t)kt0 * DK;
+  }
+  const int nk = PART ? min(nks, kpad / DK - kt0) : kpad / DK;
+  auto issue = [&](int buf, int kt) __attribute__((always_inline)) {
+    int8_t *d = lds + buf * STAGE;
+    const int k0 = kt * DK;
+#pragma unroll
+    for (int i = 0; i < LA; i++)
+      __builtin_amdgcn_global_load_lds((const void *)(ga[i] + k0), (lds_ptr_t)(d + (wave * LA + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < LB; i++)
+      __builtin_amdgcn_global_load_lds((const void *)(gb[i] + k0), (lds_ptr_t)(d + TM * DK + (wave * LB + i) * 1024), 16,
+                                       0, 0);
+  };
+  // LDS addresses of this lane's fragments of phase p in buffer 0: row lane % 32 of the wave's first row
+  // (column) block, chunk 2p + lane / 32
+  unsigned la[4], lb[4];
+  {
+    const int ra = wm * (TM / WM) + (lane & 31), rb = (MODE == GM_SWIGLU ? wn * 32 : wn * 64) + (lane & 31);
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+      la[p] = (unsigned)(uintptr_t)lds + ra * DK + (((2 * p + (lane >> 5)) ^ swz_deep(ra)) << 4);
+      lb[p] = (unsigned)(uintptr_t)lds + (TM + rb) * DK + (((2 * p + (lane >> 5)) ^ swz_deep(rb)) << 4);
+    }
+  }
+
+  v16i acc[RB][2];
+#pragma unroll
+  for (int a = 0; a < RB; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++) acc[a][b] = (v16i){};
+  v4i xa[RB], xb[2], ya[RB], yb[2];
+
+#pragma unroll
+  for (int i = 0; i < NS; i++)
+    if (i < nk) issue(i, i);
+  if (nk >= NS) wait_vmcnt<LPS * (NS - 1)>();
+  else wait_vmcnt<0>();
+  block_sync_lds();
+  // the first fragments: read and waited for in one block (the sums they go into are still zero, and so
+  // are the fragments multiplied meanwhile)
+#pragma unroll
+  for (int a = 0; a < RB; a++) ya[a] = (v4i){};
+#pragma unroll
+  for (int b = 0; b < 2; b++) yb[b] = (v4i){};
+  gemm_phase<BOFF>(acc, ya, yb, xa, xb, la[0], lb[0]);
+  int buf = 0;
+  for (int kt = 0; kt < nk; kt++) {
+    const unsigned o = buf * STAGE;
+    gemm_phase<BOFF>(acc, xa, xb, ya, yb, la[1] + o, lb[1] + o);
+    gemm_phase<BOFF>(acc, ya, yb, xa, xb, la[2] + o, lb[2] + o);
+    gemm_phase<BOFF>(acc, xa, xb, ya, yb, la[3] + o, lb[3] + o);
+    if (kt + NS <= nk) wait_vmcnt<LPS * (NS - 2)>();   // the copies of step kt + 1 (later ones stay in flight)
+    else wait_vmcnt<0>();
+    block_sync_lds();
+    if (kt + NS < nk) issue(buf, kt + NS);
+    buf = buf + 1 < NS ? buf + 1 : 0;
+    const unsigned n = buf * STAGE;
+    gemm_phase<BOFF>(acc, ya, yb, xa, xb, la[0] + n, lb[0] + n);   // after the last step: read, not used
+  }
+  // the compiler does not see the products' latency inside the asm blocks
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int a = 0; a < RB; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++) asm volatile("" : "+v"(acc[a][b]));
+  if constexpr (PART) epi_part<MODE, RB>(acc, el, M, N, part, split, m0 + wm * (TM / WM), lane);
+  else epi_end<MODE, RB, TM>(acc, epi, el, bias != nullptr, M, N, out, ldo, m0, n0, NOUT, wm * (TM / WM), lane);
+}
+
+template <int MODE, int TM, int TN, int WM, int WN, int NS>
+int launch_deep(const int8_t *A, const float *as, const int8_t *W, const float *ws, int M, int N, int kpad, float *out,
+                int ldo, const float *bias, int cls, int S, int *work) {
+  const int nout = MODE == GM_SWIGLU ? TN / 2 : TN;
+  const int mt = (M + TM - 1) / TM, nt = (N + nout - 1) / nout, blocks = 8 * mt * ((nt + 7) / 8), nkt = kpad / DK;
+  const dim3 block(64 * WM * WN);
+  g_last_splits = S;
+  if (S < 2) {
+    QH_LAUNCH(cls, (k_gemm_i8_deep<MODE, TM, TN, WM, WN, NS>), dim3(blocks), block, 0, A, as, W, ws, M, N, kpad, out,
+              ldo, bias, mt, nt, blocks, nkt, static_cast<int *>(nullptr));
+    return 0;
+  }
+  if constexpr (NS == 4) {
+    const int nks = (nkt + S - 1) / S;
+    QH_LAUNCH(cls, (k_gemm_i8_deep<MODE, TM, TN, WM, WN, NS, true>), dim3(blocks * S), block, 0, A, as, W, ws, M, N,
+              kpad, out, ldo, bias, mt, nt, blocks, nks, work);
+    QH_LAUNCH(cls, k_gemm_split_epi<MODE>, dim3((N + 255) / 256, M), dim3(256), 0, work, S, as, ws, M, N, out, ldo, bias);
+    return 0;
+  }
+  return qh::fail_msg("gemm_i8: this tile does not split K");
+}
+
+// Tile choice for kpad % 128 == 0, by the time of each in tenths of a microsecond
+// (measured on 2048, 1500, 1000, 512, 333, 200, 100 and 40 rows of the 8B and 1B
+// layers' products): a round of blocks takes a fixed part (first copies, epilogue)
+// and a part a step of 128 bytes of K,
+//   256 x 256, 8 waves, one block a CU                18.0 + 1.35 us a step and round
+//   256 x 128, 8 waves, three steps in LDS            15.0 + 0.96
+//   128 x 128, 4 waves, two steps in LDS, two a CU     6.0 + 0.50 us a block on its CU
+//   128 x 128, four steps in LDS, one a CU             8.0 + 0.49
+// the last with K split S ways where the caller lends a workspace (the S partial
+// planes written and read at 3 TB/s).  At 2048 rows, us: 8B gate|up 276 317 313
+// (256 x 256, 256 x 128, 128 x 128), QKV 61 71 65, Wo 86 52 46, down 189 126 131; 1B
+// down at 333 rows unsplit 43, split 5 ways 22.
 template <int MODE>
 int launch(const int8_t *A, const float *as, const int8_t *W, const float *ws, int M, int N, int kpad, float *out,
            int ldo, const float *bias, int cls, int *work, size_t work_bytes) {
-  if (kpad % BK == 0) {
-    if (MODE == GM_SWIGLU || (MODE == GM_RESID && kpad >= 8192))
-      return launch_pipe<MODE, 256, 128, 4, 2, 3>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, work, work_bytes);
-    if (MODE == GM_RESID)
-      return launch_pipe<MODE, 128, 128, 4, 2, 3>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, work, work_bytes);
-    return launch_pipe<MODE, 128, 128, 4, 2, 4>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, work, work_bytes);
+  if (kpad % DK == 0) {
+    const int cus = qh::num_cus() > 0 ? qh::num_cus() : 256, st = kpad / DK;
+    auto rounds = [&](int tm, int tn) {
+      const int nout = MODE == GM_SWIGLU ? tn / 2 : tn;
+      const long long tiles = (long long)((M + tm - 1) / tm) * ((N + nout - 1) / nout);
+      return (tiles + cus - 1) / cus;
+    };
+    long long cost = rounds(256, 256) * (1800 + 135 * st);       // hundredths
+    int best = 0, S = 1;
+    if (const long long c = rounds(256, 128) * (1500 + 96 * st); c < cost) { cost = c; best = 1; }
+    const long long n = rounds(128, 128);
+    if (n > 1) {
+      if (const long long c = n * (600 + 50 * st); c < cost) { cost = c; best = 2; }
+    } else {
+      const int nout = MODE == GM_SWIGLU ? 64 : 128, tiles = ((M + 127) / 128) * ((N + nout - 1) / nout);
+      if (const long long c = 800 + 49 * st; c < cost) { cost = c; best = 3; }
+      const size_t plane = (size_t)M * (MODE == GM_SWIGLU ? 2 * N : N) * 4;
+      for (int q = 2; work && q <= min(kMaxSplits, st / 4) && tiles * q <= cus && (size_t)q * plane <= work_bytes; q++) {
+        const int nks = (st + q - 1) / q;
+        if ((st + nks - 1) / nks != q) continue;                 // every split has steps
+        const long long c = 800 + 49 * nks + 150 + (long long)((2 * q + 2) * plane / 30000);
+        if (c < cost) { cost = c; best = 3; S = q; }
+      }
+    }
+    switch (best) {
+      case 0: return launch_deep<MODE, 256, 256, 2, 4, 2>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, 1, nullptr);
+      case 1: return launch_deep<MODE, 256, 128, 4, 2, 3>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, 1, nullptr);
+      case 2: return launch_deep<MODE, 128, 128, 2, 2, 2>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, 1, nullptr);
+      default: return launch_deep<MODE, 128, 128, 2, 2, 4>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, S, work);
+    }
   }
+  if (kpad % BK == 0)
+    return launch_pipe<MODE, 128, 128, 4, 2, 4>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, work, work_bytes);
   const int nout = MODE == GM_SWIGLU ? BN / 2 : BN;
   const int mt = (M + BM - 1) / BM, nt = (N + nout - 1) / nout;
   const int blocks = 8 * mt * ((nt + 7) / 8);

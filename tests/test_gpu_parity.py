@@ -533,3 +533,52 @@ def test_split_k_gemm_same_bits(Q, mode, M, N, kpad, bias):
         c = (a_s[:, None] * w_s[None, :]) * acc.astype(np.float32)
         want = init + c if mode == 1 else (c + b if bias else c)
         assert np.array_equal(o1.view(np.uint32), want.astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,M,N,kpad,bias", [
+    # one K step, two, three and five (fewer than the four in LDS, and one more); cut rows and columns
+    (0, 130, 200, 128, True), (1, 257, 300, 256, False), (2, 100, 130, 384, False), (0, 129, 3000, 640, False),
+    # 128 x 128 blocks two a CU
+    (0, 1000, 6000, 512, True), (2, 1030, 7000, 256, False),
+    # 256 x 256 blocks, whole and cut
+    (0, 2048, 6144, 256, True), (1, 2000, 4100, 1024, False), (2, 600, 7170, 384, False),
+    # 256 x 128 blocks, the last row and column tile cut
+    (1, 1800, 3900, 9728, False),
+    # K a multiple of 64 but not of 128
+    (0, 200, 300, 192, True), (1, 140, 520, 576, False), (2, 70, 90, 320, False)])
+def test_gemm_tiles_match_exact_sums(Q, mode, M, N, kpad, bias):
+    """Every tile shape of the prompt GEMM at its edges against the float32
+    operations of quant.c:79-82 (and llama.c:583-587 with the device's exact expf
+    left to a 1e-6 bound) over exact integer sums, on the rows around the tiles'
+    ends; with a workspace lent (K split where the rule splits) the same bits."""
+    import ctypes as C
+    rng = np.random.default_rng(9000 + 31 * mode + M + kpad)
+    wrows = 2 * N if mode == 2 else N
+    A = rng.integers(-127, 128, (M, kpad), dtype=np.int8)
+    W = rng.integers(-127, 128, (wrows, kpad), dtype=np.int8)
+    a_s = rng.uniform(1e-4, 1e-3, M).astype(np.float32)
+    w_s = rng.uniform(1e-4, 1e-3, wrows).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32) if bias else None
+    init = rng.standard_normal((M, N)).astype(np.float32)
+    o1, o2, splits = init.copy(), init.copy(), C.c_int(0)
+    f = Q.lib().qllama_test_gemm_split
+    f.restype = C.c_int
+    f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p,
+                  C.c_void_p, C.c_void_p, C.POINTER(C.c_int)]
+    p = lambda x: None if x is None else x.ctypes.data_as(C.c_void_p)
+    assert f(mode, p(A), p(a_s), p(W), p(w_s), M, N, kpad, p(b), p(o1), p(o2), C.byref(splits)) == 0
+    assert np.array_equal(o1.view(np.uint32), o2.view(np.uint32)), splits.value
+    rows = sorted({r for r in (0, 1, 31, 32, 63, 64, 127, 128, 129, 255, 256, 511, 1023, 1024, M // 2, M - 2, M - 1)
+                   if 0 <= r < M})
+    acc = (A[rows].astype(np.float64) @ W.T.astype(np.float64)).astype(np.float32)    # |acc| < 2^53: exact, rounded once
+    c = (a_s[rows, None] * w_s[None, :]) * acc
+    if mode == 2:
+        g, u = c[:, :N], c[:, N:]
+        want = g.astype(np.float64) / (1.0 + np.exp(-g.astype(np.float64))) * u
+        # five float32 roundings of at most 2^-24 each
+        assert np.all(np.abs(o1[rows] - want) <= 1e-6 * np.abs(want) + 1e-30)
+    else:
+        want = c + b[None, :] if bias else c
+        want = init[rows] + c if mode == 1 else want
+        assert np.array_equal(o1[rows].view(np.uint32), want.astype(np.float32).view(np.uint32))
