@@ -638,7 +638,7 @@ __device__ __forceinline__ void gemm_phase(v16i (&acc)[2][2], const v4i (&fa)[2]
 #undef DP_MM
 
 template <int MODE, int TM, int TN, int WM, int WN, int NS, bool PART = false>
-__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_i8_deep(
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_gemm_i8_deep(
     const int8_t *A, const float *as, const int8_t *W, const float *ws, int M, int N, int kpad, float *out, int ldo,
     const float *bias, int mt_count, int nt_count, int bps, int nks, int *part) {
   constexpr int NWAVE = WM * WN, RB = TM / WM / 32;
