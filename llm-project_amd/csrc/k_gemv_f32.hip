@@ -29,7 +29,8 @@ constexpr int kFK = 16;                        // k rows per tile of a panel
 constexpr int kFTile = kFC * kFK;              // floats per tile
 constexpr int kFDepth = 8;                     // groups of four tiles in flight
 
-enum { FMODE_PLAIN = 0, FMODE_RESID = 1, FMODE_RESID_BIAS = 2, FMODE_GELU_BIAS = 3 };
+enum { FMODE_PLAIN = 0, FMODE_RESID = 1, FMODE_RESID_BIAS = 2, FMODE_GELU_BIAS = 3, FMODE_SWIGLU = 4 };
+enum { FPRO_NONE = 0, FPRO_RMS = 1, FPRO_LN = 2 };
 
 // p, moved by a DPP control (row_shl:n is 0x100 + n: lane i takes lane i + n of
 // its row of 16; a quad permutation that broadcasts lane c of each quad is
@@ -189,6 +190,186 @@ __global__ __launch_bounds__(64) void k_gemv_f32(const float *x, int K, const fl
     else if (MODE == FMODE_RESID_BIAS) out[j] = out[j] + (acc + bias[j]);
     else if (MODE == FMODE_GELU_BIAS) out[j] = qd::gelu_tanh(acc + bias[j]);
     else out[j] = bias ? acc + bias[j] : acc;
+  }
+}
+
+// Two chains at once (the gate and the up panel of one column group): the other
+// chain's adds are the work between a chain's DPP adds.
+template <typename Mid>
+__device__ __forceinline__ void f_sum2(float &a0, float &a1, const float4 &p, const float4 &q, Mid mid) {
+#define F_PAIR(ctrl, e)                                                     \
+  a0 += f_dpp<ctrl>(p.e);                                                   \
+  __builtin_amdgcn_sched_barrier(0);                                        \
+  a1 += f_dpp<ctrl>(q.e);                                                   \
+  __builtin_amdgcn_sched_barrier(0)
+  a0 += p.x; a1 += q.x; a0 += p.y; a1 += q.y; a0 += p.z; a1 += q.z; a0 += p.w; a1 += q.w;
+  __builtin_amdgcn_sched_barrier(0);
+  F_PAIR(0x104, x); mid(0); F_PAIR(0x104, y); mid(1); F_PAIR(0x104, z); mid(2); F_PAIR(0x104, w); mid(3);
+  F_PAIR(0x108, x); mid(4); F_PAIR(0x108, y); mid(5); F_PAIR(0x108, z); mid(6); F_PAIR(0x108, w); mid(7);
+  F_PAIR(0x10c, x); F_PAIR(0x10c, y); F_PAIR(0x10c, z); F_PAIR(0x10c, w);
+#undef F_PAIR
+}
+
+// Product m of tile C (f_products, one at a time).
+template <int C>
+__device__ __forceinline__ float f_product1(const float4 &w, const float4 &x, int m) {
+  return m == 0 ? f_dpp<0x55 * C>(x.x) * w.x : m == 1 ? f_dpp<0x55 * C>(x.y) * w.y
+       : m == 2 ? f_dpp<0x55 * C>(x.z) * w.z : f_dpp<0x55 * C>(x.w) * w.w;
+}
+__device__ __forceinline__ void f_set(float4 &v, int m, float x) {
+  if (m == 0) v.x = x;
+  else if (m == 1) v.y = x;
+  else if (m == 2) v.z = x;
+  else v.w = x;
+}
+
+// Where a GEMV of [q | k | v] (GPT-2) also appends the new position's rows
+// (model.c:481-482) to the caches laid out [head][max_seq][head_dim].
+struct FAppend {
+  const int *d_state;
+  float *kc, *vc;
+  int dm, hd, max_seq;
+};
+
+// The GEMV over a row that each block normalizes for itself (K <= 256 * CM): rmsnorm
+// (rmsnorm.c:7-21) or LayerNorm into LDS by its four waves, while the first groups of
+// the panel's W are in flight; then wave 0 sums the panel as k_gemv_f32 does, x from
+// LDS, and the others end.  SwiGLU (swiglu.c:7-10, 36-39): the wave sums a gate panel
+// and the matching up panel, one chain's adds between the other's, and stores h.
+// Bound: the norm's serial sum, then the panel's chains; what it saves is a one-block
+// kernel and its boundaries, after which the GEMV would first wait for its loads.
+// Kernel times, against the separate kernels': K = 2048, rmsnorm + 3072 columns
+// 5.3 + 12.5 -> 15.4 us, rmsnorm + 2 x 8192 + SwiGLU 5.3 + 25.2 + 4.7 -> 26.8;
+// K = 768, LayerNorm + 2304 columns + append 7.4 + 6.4 + 1.6 -> 12.8, LayerNorm +
+// 3072 with GELU 7.4 + 8.0 -> 14.0.  One wave a block forming the norm alone: 18.2,
+// 30.0, 13.7, 15.4; four panels a block (all four waves sum, a quarter of the
+// CUs): 17.1, 30.6, 13.9, 15.8.
+constexpr int kFNW = 4;           // waves per block, for the norm; wave 0 then sums the panel
+
+template <int MODE, int PRO, int CM, int kFD>
+__global__ __launch_bounds__(64 * kFNW) void k_gemv_f32_norm(const float *x, int K, const float *gamma,
+                                                            const float *beta, float eps, const float *W, int N,
+                                                            float *out, const float *bias, FAppend ap) {
+  constexpr int NP = MODE == FMODE_SWIGLU ? 2 : 1, NT = 64 * kFNW;
+  __shared__ __attribute__((aligned(16))) float xs[NT * CM];
+  __shared__ qd::SeqScratch seq;
+  __shared__ float red[kFNW];
+  const int lane = threadIdx.x & 63, s = (lane >> 2) & 3, c = lane & 3, j0 = threadIdx.x * CM;
+  const int kt = (K + kFK - 1) / kFK, ng = (kt + 3) / 4;               // tiles; groups of four, the last perhaps short
+  const int np = (N + kFC - 1) / kFC;
+  const int panel = blockIdx.x;
+  const bool chains = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0;
+  float y[CM], gm[CM], be[PRO == FPRO_LN ? CM : 1];
+  qd::rmsnorm_load<CM>(x, K, gamma, y, gm);
+  if constexpr (PRO == FPRO_LN) {
+#pragma unroll
+    for (int i = 0; i < CM; i++) be[i] = j0 + i < K ? beta[j0 + i] : 0.0f;
+  }
+  __builtin_amdgcn_sched_barrier(0);          // the row first: loads return in order
+  __amdgpu_buffer_rsrc_t rw[NP];
+#pragma unroll
+  for (int n = 0; n < NP; n++) {
+    const float *Wp = W + ((size_t)panel + (size_t)n * np) * kt * kFTile;
+    rw[n] = __builtin_amdgcn_make_buffer_rsrc((void *)Wp, (short)0, chains ? kt * kFTile * 4 : 0, 0x00020000);
+  }
+  const int vw = lane * 16;
+  float4 w[kFD][NP][4], xv[kFD];
+  auto loadw = [&](int d, int g, int t) __attribute__((always_inline)) {       // past the panel's end: reads 0, no traffic
+#pragma unroll
+    for (int n = 0; n < NP; n++) w[d][n][t] = f_load16(rw[n], vw + t * kFTile * 4, g * 4 * kFTile * 4);
+  };
+  auto loadx = [&](int d, int g) __attribute__((always_inline)) {              // groups past the last: the last again
+    xv[d] = *reinterpret_cast<const float4 *>(&xs[min(g, ng - 1) * 4 * kFK + 16 * c + 4 * s]);
+  };
+#pragma unroll
+  for (int d = 0; d < kFD; d++) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) loadw(d, d, t);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (PRO == FPRO_LN) qd::layernorm_apply<NT, CM>(x, K, eps, y, gm, be, xs, &red[0], seq);
+  else (void)qd::rmsnorm_apply<NT, CM>(x, K, eps, y, gm, red, seq);
+#pragma unroll
+  for (int i = 0; i < CM; i += 4) {
+    float4 v = make_float4(y[i], y[i + 1], y[i + 2], y[i + 3]);
+    if (j0 + i >= K) v.x = 0.0f;                // LayerNorm leaves garbage past K
+    if (j0 + i + 1 >= K) v.y = 0.0f;
+    if (j0 + i + 2 >= K) v.z = 0.0f;
+    if (j0 + i + 3 >= K) v.w = 0.0f;
+    *reinterpret_cast<float4 *>(&xs[j0 + i]) = v;
+  }
+  qd::lds_sync();                               // the last barrier
+  if (!chains) return;
+#pragma unroll
+  for (int d = 0; d < kFD; d++) loadx(d, d);
+
+  float acc[NP];
+#pragma unroll
+  for (int n = 0; n < NP; n++) acc[n] = 0.0f;
+  // one tile's sums, with the products of the next formed and `more` requested meanwhile
+  float4 p[2][NP];
+  auto tile = [&](auto cv, auto &cur, auto &nxt, const float4 (&wn)[NP][4], const float4 &xn, auto more)
+      __attribute__((always_inline)) {
+    constexpr int C = decltype(cv)::value;      // tile of its group that `nxt` is of
+    if constexpr (NP == 1) {
+      f_sum(acc[0], cur[0], [&](int i) __attribute__((always_inline)) {
+        f_set(nxt[0], i, f_product1<C>(wn[0][C], xn, i));
+        more(i);
+      });
+    } else {
+      f_sum2(acc[0], acc[NP - 1], cur[0], cur[NP - 1], [&](int i) __attribute__((always_inline)) {
+        f_set(nxt[i >> 2], i & 3, f_product1<C>(wn[i >> 2][C], xn, i & 3));
+        if (i < 4) more(i);
+      });
+    }
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  using C2 = std::integral_constant<int, 2>;
+  using C3 = std::integral_constant<int, 3>;
+  auto none = [](int) {};
+#pragma unroll
+  for (int n = 0; n < NP; n++) p[0][n] = f_products<0>(w[0][n][0], xv[0]);
+  int g0 = 0;
+  for (; g0 + kFD < ng; g0 += kFD) {
+#pragma unroll
+    for (int d = 0; d < kFD; d++) {
+      const int g = g0 + d + kFD, e = (d + 1) % kFD;
+      tile(C1(), p[0], p[1], w[d], xv[d], none);
+      tile(C2(), p[1], p[0], w[d], xv[d], [&](int i) __attribute__((always_inline)) { if (i == 1) loadw(d, g, 0); });
+      tile(C3(), p[0], p[1], w[d], xv[d], [&](int i) __attribute__((always_inline)) { if (i == 1) loadw(d, g, 1); });
+      tile(C0(), p[1], p[0], w[e], xv[e], [&](int i) __attribute__((always_inline)) {
+        if (i == 1) loadw(d, g, 2);
+        if (i == 2) loadw(d, g, 3);
+        if (i == 3) loadx(d, g);
+      });
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < kFD; d++) {               // the last 1 .. kFD groups (a short one's missing tiles are 0)
+    if (g0 + d < ng) {
+      const int e = (d + 1) % kFD;
+      tile(C1(), p[0], p[1], w[d], xv[d], none);
+      tile(C2(), p[1], p[0], w[d], xv[d], none);
+      tile(C3(), p[0], p[1], w[d], xv[d], none);
+      tile(C0(), p[1], p[0], w[e], xv[e], none);
+    }
+  }
+  const int j = panel * kFC + 4 * (lane >> 4) + c;
+  if (s == 0 && j < N) {
+    if (MODE == FMODE_SWIGLU) {
+      const float z = acc[0], sg = 1.0f / (1.0f + qd::expf_glibc(-z));
+      out[j] = (z * sg) * acc[NP - 1];
+    } else if (MODE == FMODE_GELU_BIAS) {
+      out[j] = qd::gelu_tanh(acc[0] + bias[j]);
+    } else {
+      const float v = bias ? acc[0] + bias[j] : acc[0];
+      out[j] = v;
+      if (PRO == FPRO_LN && ap.d_state && j >= ap.dm) {
+        const int i = j < 2 * ap.dm ? j - ap.dm : j - 2 * ap.dm, h = i / ap.hd;
+        (j < 2 * ap.dm ? ap.kc : ap.vc)[((size_t)h * ap.max_seq + ap.d_state[0]) * ap.hd + (i - h * ap.hd)] = v;
+      }
+    }
   }
 }
 
@@ -444,6 +625,38 @@ extern "C" int qhip_gemv_f32(int mode, int cls, const float *x, int K, const flo
     default: QH_LAUNCH(cls, (k_gemv_f32<FMODE_GELU_BIAS, kFDepth>), grid, block, 0, x, K, W, N, out, bias); break;
   }
   return 0;
+}
+
+// Whether qhip_gemv_f32_norm takes this shape: panels that do not mix gate and up
+// columns (SwiGLU), at most 1024 of them (four blocks a CU: every block forms the
+// norm at once, none waits for another's to end), and K up to 2048 (measured ahead
+// of the separate kernels from 48 to 2048, at the head of this kernel; a longer row's
+// weights stream for much longer than the kernel that this saves).
+extern "C" int qhip_gemv_f32_norm_ok(int mode, int K, int N) {
+  return K >= 1 && K <= 64 * kFNW * 8 && (mode != FMODE_SWIGLU || N % kFC == 0) && (N + kFC - 1) / kFC <= 1024;
+}
+
+extern "C" int qhip_gemv_f32_norm(int pro, int mode, int cls, const float *x, int K, const float *gamma,
+                                  const float *beta, float eps, const float *W, int N, float *out, const float *bias,
+                                  const int *d_state, float *kc, float *vc, int hd, int max_seq) {
+  if (!qhip_gemv_f32_norm_ok(mode, K, N) || N <= 0) return qh::fail_msg("gemv_f32_norm: unsupported shape");
+  const int np = (N + kFC - 1) / kFC;
+  const dim3 grid(np), block(64 * kFNW);
+  const FAppend ap{d_state, kc, vc, N / 3, hd, max_seq};
+#define F_NORM(MODE, PRO, FD)                                                                                         \
+  do {                                                                                                                \
+    if (K <= 64 * kFNW * 4) QH_LAUNCH(cls, (k_gemv_f32_norm<MODE, PRO, 4, FD>), grid, block, 0, x, K, gamma, beta,   \
+                                      eps, W, N, out, bias, ap);                                                     \
+    else QH_LAUNCH(cls, (k_gemv_f32_norm<MODE, PRO, 8, FD>), grid, block, 0, x, K, gamma, beta, eps, W, N, out, bias, \
+                   ap);                                                                                               \
+    return 0;                                                                                                         \
+  } while (0)
+  if (pro == FPRO_RMS && mode == FMODE_PLAIN) F_NORM(FMODE_PLAIN, FPRO_RMS, kFDepth);
+  if (pro == FPRO_RMS && mode == FMODE_SWIGLU) F_NORM(FMODE_SWIGLU, FPRO_RMS, 5);
+  if (pro == FPRO_LN && mode == FMODE_PLAIN) F_NORM(FMODE_PLAIN, FPRO_LN, kFDepth);
+  if (pro == FPRO_LN && mode == FMODE_GELU_BIAS && bias) F_NORM(FMODE_GELU_BIAS, FPRO_LN, kFDepth);
+#undef F_NORM
+  return qh::fail_msg("gemv_f32_norm: bad mode");
 }
 
 // Floats of a (K, N) matrix in the panel layout.

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "qdev_math.h"
+#include "qdev_norm.h"
 #include "qdev_seqsum.h"
 #include "qhip.h"
 #include "qhip_internal.h"
@@ -21,11 +22,7 @@ __global__ void k_gpt_embed(const float *wte, const float *wpe, int dm, const in
   x[j] = wte[(size_t)d_in[pos] * dm + j] + wpe[(size_t)pos * dm + j];
 }
 
-// layernorm.c:8-38 for one row, one block of NT threads (thread t holds
-// elements [t*CM, t*CM + CM)):
-//   mean = (sum_j x_j, in order) / cols       -- a serial chain (signed terms), one lane
-//   var  = (sum_j (x_j - mean)^2, in order) / cols   -- exact parallel sum (qdev_seqsum.h)
-//   y_j  = ((x_j - mean) * (1 / sqrtf(var + eps))) * gamma_j + beta_j
+// layernorm.c:8-38 for one row, one block of NT threads (qdev_norm.h)
 template <int NT, int CM>
 __global__ __launch_bounds__(NT) void k_layernorm_f32(const float *x, int dm, const float *gamma, const float *beta,
                                                       float eps, float *y) {
@@ -40,57 +37,10 @@ __global__ __launch_bounds__(NT) void k_layernorm_f32(const float *x, int dm, co
     ga[c] = j0 + c < dm ? gamma[j0 + c] : 0.0f;       // requested now, used at the end
     be[c] = j0 + c < dm ? beta[j0 + c] : 0.0f;
   }
+  qd::layernorm_apply<NT, CM>(x, dm, eps, v, ga, be, xs, &mean_s, seq);
 #pragma unroll
-  for (int c = 0; c < CM; c++) xs[j0 + c] = v[c];
-  qd::lds_sync();
-  if (threadIdx.x == 0) {
-    // the chain over exactly dm terms, 16 at a time from LDS with the next 16
-    // requested before the current ones are added (the reads land while the
-    // adds run); a tail of dm % 16 terms one by one
-    const float4 *x4 = reinterpret_cast<const float4 *>(xs);
-    const int n16 = dm / 16;
-    float s = 0.0f;
-    float4 a[4], b[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) a[u] = n16 > 0 ? x4[u] : make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int i = 0; i < n16; i++) {
-      const int nx = i + 1 < n16 ? i + 1 : i;
-#pragma unroll
-      for (int u = 0; u < 4; u++) b[u] = x4[4 * nx + u];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        s += a[u].x;
-        s += a[u].y;
-        s += a[u].z;
-        s += a[u].w;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) a[u] = b[u];
-    }
-    for (int j = 16 * n16; j < dm; j++) s += xs[j];
-    mean_s = s / (float)dm;
-  }
-  qd::lds_sync();
-  const float mean = mean_s;
-  float sq[CM];
-#pragma unroll
-  for (int c = 0; c < CM; c++) {
-    const float d = v[c] - mean;
-    sq[c] = j0 + c < dm ? d * d : 0.0f;
-  }
-  float var = qd::seq_sum_nonneg<NT, CM>(sq, dm, seq, [&](int i) {
-    const float d = x[i] - mean;
-    return d * d;
-  });
-  var = var / (float)dm;
-  const float inv_std = 1.0f / sqrtf(var + eps);
-#pragma unroll
-  for (int c = 0; c < CM; c++) {
-    if (j0 + c < dm) {
-      const float t = (v[c] - mean) * inv_std;
-      y[j0 + c] = t * ga[c] + be[c];
-    }
-  }
+  for (int c = 0; c < CM; c++)
+    if (j0 + c < dm) y[j0 + c] = v[c];
 }
 
 // The new position's k and v rows (model.c:481-482) into the per-layer caches

@@ -107,6 +107,68 @@ __device__ __forceinline__ float rmsnorm_apply_fast(int n, float eps, float (&y)
   return (mx > 0.0f) ? mx / 127.0f : 1.0f;
 }
 
+// LayerNorm (layernorm.c:8-38) of one row by one block of NT threads, v[], ga[] and
+// be[] holding the row's values, gammas and betas of elements [t*CM, t*CM + CM) of
+// thread t (0 past n); v[] receives the result.
+//   mean = (sum_j x_j, in order) / n       -- a serial chain (signed terms), one lane
+//   var  = (sum_j (x_j - mean)^2, in order) / n   -- exact parallel sum (qdev_seqsum.h)
+//   y_j  = ((x_j - mean) * (1 / sqrtf(var + eps))) * gamma_j + beta_j
+// xs: NT*CM floats of LDS, 16-byte aligned.
+template <int NT, int CM>
+__device__ __forceinline__ void layernorm_apply(const float *x, int n, float eps, float (&v)[CM], const float (&ga)[CM],
+                                                const float (&be)[CM], float *xs, float *mean_s, SeqScratch &seq) {
+  const int j0 = threadIdx.x * CM;
+#pragma unroll
+  for (int c = 0; c < CM; c++) xs[j0 + c] = v[c];
+  lds_sync();
+  if (threadIdx.x == 0) {
+    // the chain over exactly n terms, 16 at a time from LDS with the next 16
+    // requested before the current ones are added (the reads land while the
+    // adds run); a tail of n % 16 terms one by one
+    const float4 *x4 = reinterpret_cast<const float4 *>(xs);
+    const int n16 = n / 16;
+    float s = 0.0f;
+    float4 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) a[u] = n16 > 0 ? x4[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < n16; i++) {
+      const int nx = i + 1 < n16 ? i + 1 : i;
+#pragma unroll
+      for (int u = 0; u < 4; u++) b[u] = x4[4 * nx + u];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        s += a[u].x;
+        s += a[u].y;
+        s += a[u].z;
+        s += a[u].w;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) a[u] = b[u];
+    }
+    for (int j = 16 * n16; j < n; j++) s += xs[j];
+    *mean_s = s / (float)n;
+  }
+  lds_sync();
+  const float mean = *mean_s;
+  float sq[CM];
+#pragma unroll
+  for (int c = 0; c < CM; c++) {
+    const float d = v[c] - mean;
+    sq[c] = j0 + c < n ? d * d : 0.0f;
+  }
+  float var = seq_sum_nonneg<NT, CM>(sq, n, seq, [&](int i) {
+    const float d = x[i] - mean;
+    return d * d;
+  });
+  var = var / (float)n;
+  const float inv_std = 1.0f / sqrtf(var + eps);
+#pragma unroll
+  for (int c = 0; c < CM; c++) {
+    const float t = (v[c] - mean) * inv_std;
+    v[c] = t * ga[c] + be[c];
+  }
+}
+
 // Both steps: y[] receives this thread's normalized values.
 template <int NT, int CM>
 __device__ __forceinline__ float rmsnorm_row(const float *xr, int n, const float *gamma, float eps, float (&y)[CM],

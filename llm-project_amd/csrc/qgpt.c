@@ -324,16 +324,27 @@ static GDev *gdev_create(const GPT *m) {
 static int enqueue_gpt_step(const GDev *g) {
   const size_t per = (size_t)g->max_seq * g->dm;
   const float scale = 1.0f / sqrtf((float)g->hd);           // model.c:460
+  const int nq = qhip_gemv_f32_norm_ok(0, g->dm, 3 * g->dm), n1 = qhip_gemv_f32_norm_ok(3, g->dm, g->ff);
   int rc = qhip_gpt_embed(g->wte, g->wpe, g->dm, g->d_in, g->d_state, g->x);
   for (int l = 0; l < g->L && !rc; l++) {
     float *kc = g->kbase + (size_t)l * per, *vc = g->vbase + (size_t)l * per;
-    rc |= qhip_layernorm_f32(g->x, g->dm, g->g1[l], g->be1[l], GPT_LN_EPS, g->xn);
-    rc |= qhip_gemv_f32(0, 2, g->xn, g->dm, g->wqkv[l], 3 * g->dm, g->qkv, g->bqkv[l]);
-    rc |= qhip_gpt_kv_append(g->qkv, g->dm, g->hd, g->max_seq, g->d_state, kc, vc);
+    if (nq) {                 // LayerNorm and the cache append inside the QKV GEMV
+      rc |= qhip_gemv_f32_norm(2, 0, 2, g->x, g->dm, g->g1[l], g->be1[l], GPT_LN_EPS, g->wqkv[l], 3 * g->dm, g->qkv,
+                               g->bqkv[l], g->d_state, kc, vc, g->hd, g->max_seq);
+    } else {
+      rc |= qhip_layernorm_f32(g->x, g->dm, g->g1[l], g->be1[l], GPT_LN_EPS, g->xn);
+      rc |= qhip_gemv_f32(0, 2, g->xn, g->dm, g->wqkv[l], 3 * g->dm, g->qkv, g->bqkv[l]);
+      rc |= qhip_gpt_kv_append(g->qkv, g->dm, g->hd, g->max_seq, g->d_state, kc, vc);
+    }
     rc |= qhip_attention_div(g->qkv, kc, vc, g->d_state, g->nh, g->nh, g->hd, g->max_seq, scale, g->scores, g->o);
     rc |= qhip_gemv_f32(2, 6, g->o, g->dm, g->wo[l], g->dm, g->x, g->bo[l]);
-    rc |= qhip_layernorm_f32(g->x, g->dm, g->g2[l], g->be2[l], GPT_LN_EPS, g->xn);
-    rc |= qhip_gemv_f32(3, 7, g->xn, g->dm, g->w1[l], g->ff, g->h, g->bf1[l]);
+    if (n1) {
+      rc |= qhip_gemv_f32_norm(2, 3, 7, g->x, g->dm, g->g2[l], g->be2[l], GPT_LN_EPS, g->w1[l], g->ff, g->h, g->bf1[l],
+                               NULL, NULL, NULL, 0, 0);
+    } else {
+      rc |= qhip_layernorm_f32(g->x, g->dm, g->g2[l], g->be2[l], GPT_LN_EPS, g->xn);
+      rc |= qhip_gemv_f32(3, 7, g->xn, g->dm, g->w1[l], g->ff, g->h, g->bf1[l]);
+    }
     rc |= qhip_gemv_f32(2, 9, g->h, g->ff, g->w2[l], g->dm, g->x, g->bf2[l]);
   }
   if (!rc) rc |= qhip_layernorm_f32(g->x, g->dm, g->lnf_g, g->lnf_b, GPT_LN_EPS, g->xn);

@@ -253,6 +253,14 @@ size_t qhip_panels_f32_size(int K, int N);
 int qhip_to_panels_f32(const float *src, int K, int N, float *dst);
 // mode 0: out = c (+ bias); 1: out += c; 2: out = out + (c + bias); 3: out = gelu(c + bias).
 int qhip_gemv_f32(int mode, int cls, const float *x, int K, const float *W, int N, float *out, const float *bias);
+// The GEMV over a row normalized inside it: pro 1 rmsnorm (gamma, eps), 2 LayerNorm
+// (gamma, beta, eps); mode 0 plain (+ bias; pro 2 with d_state: [q | k | v], whose k and
+// v also go to row d_state[0] of kc and vc, [head][max_seq][hd]), 3 GELU(c + bias), 4
+// SwiGLU (W has 2N columns, gate then up; out = N values of h).
+int qhip_gemv_f32_norm_ok(int mode, int K, int N);
+int qhip_gemv_f32_norm(int pro, int mode, int cls, const float *x, int K, const float *gamma, const float *beta,
+                       float eps, const float *W, int N, float *out, const float *bias, const int *d_state, float *kc,
+                       float *vc, int hd, int max_seq);
 int qhip_gemv_f32_max_k(void);
 int qhip_embed_f32(const float *wte, int dm, const int *d_in, const int *d_state, float *x);
 int qhip_rmsnorm_f32(const float *x, int dm, const float *gamma, float eps, float *y);

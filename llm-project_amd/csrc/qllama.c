@@ -1098,17 +1098,28 @@ static FDev *fdev_upload(const LlamaModel *m) {
 // llama.c:296-362 for the token at d_in[d_state[0]]
 static int enqueue_step_f32(const FDev *f, const KVDev *kd) {
   const size_t per = (size_t)f->max_seq * f->kvd;
+  const int nq = qhip_gemv_f32_norm_ok(0, f->dm, f->nqkv), nh = qhip_gemv_f32_norm_ok(4, f->dm, f->dff);
   int rc = qhip_embed_f32(f->wte, f->dm, f->d_in, f->d_state, f->x);
   for (int l = 0; l < f->L && !rc; l++) {
     float *kc = kd->kbase + (size_t)l * per, *vc = kd->vbase + (size_t)l * per;
-    rc |= qhip_rmsnorm_f32(f->x, f->dm, f->g_attn[l], f->eps, f->xn);
-    rc |= qhip_gemv_f32(0, 2, f->xn, f->dm, f->wqkv[l], f->nqkv, f->qkv, f->bqkv[l]);
+    if (nq) {                 // rmsnorm inside the QKV GEMV
+      rc |= qhip_gemv_f32_norm(1, 0, 2, f->x, f->dm, f->g_attn[l], NULL, f->eps, f->wqkv[l], f->nqkv, f->qkv,
+                               f->bqkv[l], NULL, NULL, NULL, 0, 0);
+    } else {
+      rc |= qhip_rmsnorm_f32(f->x, f->dm, f->g_attn[l], f->eps, f->xn);
+      rc |= qhip_gemv_f32(0, 2, f->xn, f->dm, f->wqkv[l], f->nqkv, f->qkv, f->bqkv[l]);
+    }
     rc |= qhip_attention_rope(f->qkv, kc, vc, f->d_state, f->H, f->KVH, f->hd, f->max_seq, f->attn_scale,
                               f->rope_cos, f->rope_sin, f->scores, f->o, NULL);
     rc |= qhip_gemv_f32(1, 6, f->o, f->qd, f->wo[l], f->dm, f->x, NULL);
-    rc |= qhip_rmsnorm_f32(f->x, f->dm, f->g_ffn[l], f->eps, f->xn);
-    rc |= qhip_gemv_f32(0, 7, f->xn, f->dm, f->wgu[l], 2 * f->dff, f->gu, NULL);
-    rc |= qhip_swiglu_f32(f->gu, f->dff, f->h);
+    if (nh) {                 // rmsnorm and SwiGLU inside the gate|up GEMV
+      rc |= qhip_gemv_f32_norm(1, 4, 7, f->x, f->dm, f->g_ffn[l], NULL, f->eps, f->wgu[l], f->dff, f->h, NULL, NULL,
+                               NULL, NULL, 0, 0);
+    } else {
+      rc |= qhip_rmsnorm_f32(f->x, f->dm, f->g_ffn[l], f->eps, f->xn);
+      rc |= qhip_gemv_f32(0, 7, f->xn, f->dm, f->wgu[l], 2 * f->dff, f->gu, NULL);
+      rc |= qhip_swiglu_f32(f->gu, f->dff, f->h);
+    }
     rc |= qhip_gemv_f32(1, 9, f->h, f->dff, f->wd[l], f->dm, f->x, NULL);
   }
   if (!rc) rc |= qhip_rmsnorm_f32(f->x, f->dm, f->g_final, f->eps, f->xn);

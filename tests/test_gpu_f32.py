@@ -80,6 +80,27 @@ def test_f32_gemv_group_edges_match_oracle(Q, K):
         ref.close()
 
 
+@pytest.mark.parametrize("dm,dff", [(1, 16), (63, 48), (1023, 32), (1024, 33), (1025, 1040), (2047, 16), (2048, 64),
+                                    (2049, 64), (64, 16384), (64, 16400)])
+def test_f32_norm_in_gemv_edges_match_oracle(Q, dm, dff):
+    """The decode GEMVs that normalize their row themselves, where that changes
+    form: rows of one float, around 1024 (elements a thread) and 2048 (separate
+    kernels), gate|up widths that are not whole panels (separate SwiGLU) and
+    around 1024 panels: bit for bit against the oracle."""
+    cfg = [33, dm, 2, 2, 1, 16, dff, 16]
+    ref = O.FModel(cfg, 10000.0, seed=dm + dff)
+    try:
+        g = gpu_model(Q, ref, cfg, 10000.0)
+        try:
+            for t in [1, 5, 32]:
+                r = ref.step(t).copy()
+                assert np.array_equal(bits(g.step(t)), bits(r)), (dm, dff, t)
+        finally:
+            g.close()
+    finally:
+        ref.close()
+
+
 @pytest.mark.parametrize("rows,dff,vocab", [(1, 33, 70), (5, 64, 17), (9, 100, 130), (40, 31, 64), (70, 95, 2100),
                                             (300, 66, 16384)])
 def test_f32_forward_tile_edges_match_oracle(Q, rows, dff, vocab):

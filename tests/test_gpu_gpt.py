@@ -121,6 +121,23 @@ def test_gpt_cache_takes_another_model(Q):
         b.close()
 
 
+@pytest.mark.parametrize("dm,heads,ff", [(8, 2, 5), (72, 3, 100), (1020, 5, 33), (1032, 4, 48), (2048, 16, 17),
+                                         (2064, 8, 64), (64, 1, 16400)])
+def test_gpt_layernorm_in_gemv_edges_match_oracle(Q, dm, heads, ff):
+    """LayerNorm and the cache append inside the decode GEMVs, around the row
+    lengths and widths where they change form or leave it to the separate kernels,
+    up to the last position of the cache: bit for bit against the oracle."""
+    om = O.GPTModel([40, dm, heads, 2, ff, 4], seed=dm)
+    dec = Q.GPTDecoder(_host_model(Q, om))
+    try:
+        for t in [3, 39, 0, 7]:
+            r = om.step(t).copy()
+            assert np.array_equal(bits(dec.step(t)), bits(r)), (dm, heads, ff, t)
+    finally:
+        dec.close()
+        om.close()
+
+
 def test_gpt_weights_changed_in_place_need_a_refresh(Q):
     """The device copy of a cache's weights is made at creation (and when the
     step is given another model): weights edited in place are not seen until
