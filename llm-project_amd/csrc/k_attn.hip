@@ -1227,58 +1227,122 @@ template <> struct MxShape<16> {
   __device__ static int col(int r, int l) { return 16 * (r >> 2) + (l & 15); }
 };
 
+// Buffer accesses of `n` floats from base: a byte offset a lane, one per wave, and
+// the range check (past n: reads 0, stores nothing).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mx_rsrc(const float *base, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, n * 4, 0x00020000);
+}
+__device__ __forceinline__ float4 mx_load16(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  const v4u t = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
+  return make_float4(__uint_as_float(t.x), __uint_as_float(t.y), __uint_as_float(t.z), __uint_as_float(t.w));
+}
+__device__ __forceinline__ float mx_load4(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
+}
+__device__ __forceinline__ void mx_store4(__amdgpu_buffer_rsrc_t r, int off, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0);
+}
+
 // Scores: block (KV head, rbq rows, i.e. 32 pairs, 8 * NP keys) of four waves;
 // wave v takes pairs NP * (v % (32 / NP)) .. +NP-1 and keys j0 + 64 * (v / (32 /
 // NP)) .. +63 (lane l supplies key j0 + l, lane l % NP the pair) and forms the
-// dots over d in order for its NP x 64 (pair, key) elements at once.  Each lane
-// reads its q and K rows a whole 128-byte line at a time (32 dims), so a line
-// is fetched once while it is in the L1.
-// Held to 4 waves per SIMD (128 registers; 134 unbounded, i.e. 3 waves): the
-// issue rate of a SIMD's MFMAs and adds rises with its waves (365 against 378
-// us per layer at the 8B shape, 2048 rows).
+// dots over d in order for its NP x 64 (pair, key) elements at once.  The pairs' q
+// rows are the same for the four waves and come from LDS; a lane reads its key's
+// row half a 128-byte line at a time, two halves ahead of the one being added
+// (smaller steps would fetch a line from L2 once for each of them).
+// Bound: a SIMD's issue of MFMAs and adds, which do not overlap (64.5 ns per 2048
+// products: 264 us at the 8B shape, 2048 rows).  Held to 4 waves per SIMD (128
+// registers): the issue rate rises with a SIMD's waves.  383 -> 345 us at that
+// shape and 22.1 -> 19.2 at 333 rows of hd 64 against q and K both from memory a
+// line at a time and each element's address and test formed on its own (about 600
+// instructions a wave, many of them multiplies, after 4096 adds).
 template <int HD, int NP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_pf_scores_mx(const float *q, const float *kc, int R, int p0, int H,
                                                       int KVH, int max_seq, float scale, float *w, int Tp) {
   typedef MxShape<NP> S;
   typedef typename S::tile tile;
-  constexpr int CH = HD % 32 == 0 ? 32 : 16, NQ = CH / 4;           // dims per step, float4 loads per row
-  static_assert(HD % CH == 0, "whole steps");
   const int kvh = blockIdx.x, G = H / KVH;
   const MxPairs P(G);
   const int r0 = blockIdx.y * P.rbq, rend = min(R, r0 + P.rbq);
   const int jvis = p0 + rend - 1;                                    // last key any row here sees
   const int lane = threadIdx.x & 63, wv_ = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int pb = NP * (wv_ % (32 / NP));
+  if ((int)(blockIdx.z * 8 * NP) > jvis) return;                     // uniform for the block
   const int jw = blockIdx.z * 8 * NP + 64 * (wv_ / (32 / NP));
+  const __amdgpu_buffer_rsrc_t rk = mx_rsrc(kc + (size_t)kvh * max_seq * HD, max_seq * HD);
+  const int ok = min(jw + lane, jvis) * HD * 4;
+  constexpr int NH = HD / 16;
+  static_assert(HD % 16 == 0, "whole halves of a line");
+  float4 kb[2][4];
+  auto kload = [&](auto bv, int h) __attribute__((always_inline)) {  // 64 bytes of the lane's key: dims 16h .. 16h+15
+#pragma unroll
+    for (int i = 0; i < 4; i++) kb[decltype(bv)::value][i] = mx_load16(rk, ok + 16 * i, 64 * h);
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  kload(B0(), 0);
+  kload(B1(), 1);
+  // the block's 32 q rows, [4 dims][pair]
+  __shared__ float4 qs[HD / 4][32];
+  {
+    const int pq = threadIdx.x & 31, gq = min(P.head(pq), G - 1), rq = min(r0 + P.row(pq), R - 1);
+    const float4 *qr = reinterpret_cast<const float4 *>(q + ((size_t)rq * H + kvh * G + gq) * HD);
+    float4 t[(HD / 4 + 7) / 8];
+#pragma unroll
+    for (int c = 0; c < HD / 4; c += 8) t[c / 8] = qr[min(c + (int)(threadIdx.x >> 5), HD / 4 - 1)];
+#pragma unroll
+    for (int c = 0; c < HD / 4; c += 8) qs[min(c + (int)(threadIdx.x >> 5), HD / 4 - 1)][pq] = t[c / 8];
+  }
+  __syncthreads();
   if (jw > jvis) return;                                             // uniform for the wave
-  const int pa = pb + (lane & (NP - 1)), ga = min(P.head(pa), G - 1), ra = min(r0 + P.row(pa), R - 1);
-  const float4 *qr = reinterpret_cast<const float4 *>(q + ((size_t)ra * H + kvh * G + ga) * HD);
-  const float4 *kr = reinterpret_cast<const float4 *>(kc + ((size_t)kvh * max_seq + min(jw + lane, jvis)) * HD);
+  const int pl = pb + (lane & (NP - 1));
   tile s = {};
-  auto add = [&](float a, float b) {
+  auto add = [&](float a, float b) __attribute__((always_inline)) {
     s += S::outer(a, b);
     __builtin_amdgcn_sched_barrier(0);                               // one product tile live at a time
   };
+  float4 qa = qs[0][pl];
+  auto half = [&](auto bv, int h) __attribute__((always_inline)) {
+    constexpr int B = decltype(bv)::value;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float4 qc = qa;
+      qa = qs[min(4 * h + i + 1, HD / 4 - 1)][pl];
+      __builtin_amdgcn_sched_barrier(0);
+      add(qc.x, kb[B][i].x);
+      add(qc.y, kb[B][i].y);
+      add(qc.z, kb[B][i].z);
+      add(qc.w, kb[B][i].w);
+    }
+    if constexpr (NH % 2) {                                          // one half a turn: the other moves up
+#pragma unroll
+      for (int i = 0; i < 4; i++) kb[0][i] = kb[1][i];
+    }
+    kload(std::integral_constant<int, NH % 2 ? 1 : B>(), h + 2);     // past the row: the next key's, or 0; not added
+    __builtin_amdgcn_sched_barrier(0);
+  };
 #pragma unroll 1
-  for (int c = 0; c < HD / 4; c += NQ) {
-    float4 qa[NQ], kb[NQ];
-#pragma unroll
-    for (int i = 0; i < NQ; i++) {
-      qa[i] = qr[c + i];
-      kb[i] = kr[c + i];
-    }
-#pragma unroll
-    for (int i = 0; i < NQ; i++) {
-      add(qa[i].x, kb[i].x);
-      add(qa[i].y, kb[i].y);
-      add(qa[i].z, kb[i].z);
-      add(qa[i].w, kb[i].w);
-    }
+  for (int h = 0; h < NH; h += 2 - NH % 2) {
+    half(B0(), h);
+    if constexpr (NH % 2 == 0) half(B1(), h + 1);
   }
+  // Lane p of the first NP holds where pair p's row starts and the last key it
+  // sees (-1: no such pair); the elements' lanes fetch it from there.  What is not
+  // to be written goes past the buffer's end.
+  const __amdgpu_buffer_rsrc_t rw = mx_rsrc(w + (size_t)kvh * G * R * Tp, G * R * Tp);
+  const int gp = P.head(pl), rp = r0 + P.row(pl);
+  const int ow = (min(gp, G - 1) * R + min(rp, R - 1)) * Tp * 4, lim = gp < G && rp < R ? p0 + rp : -1;
+  constexpr int NR = 4 * NP / (NP == 32 ? 8 : 16);                   // rows a lane holds of
 #pragma unroll
-  for (int r = 0; r < NP; r++) {
-    const int p = pb + S::row(r, lane), g = P.head(p), row = r0 + p - g * P.rbq, j = jw + S::col(r, lane);
-    if (g < G && row < R && j <= p0 + row) w[((size_t)(kvh * G + g) * R + row) * Tp + j] = s[r] * scale;
+  for (int r = 0; r < NR; r++) {
+    const int from = 4 * S::row(r, lane);
+    const int orow = __builtin_amdgcn_ds_bpermute(from, ow), last = __builtin_amdgcn_ds_bpermute(from, lim);
+#pragma unroll
+    for (int c = 0; c < NP / NR; c++) {
+      const int e = NR * c + r, j = jw + S::col(e, lane);
+      mx_store4(rw, j <= last ? orow + 4 * j : (int)0x80000000, s[e] * scale);
+    }
   }
 }
 
@@ -1288,8 +1352,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // w[pair][t] * V[t][d] of the wave's NP x 64 elements are added at once (NP
 // adds a lane per key: with NP = 16 the longest rows' waves, which bound the
 // kernel, carry half the adds of NP = 32).  Keys up to the block's first row's
-// last are seen by every pair: they go 8 a chunk, one chunk in flight while the
-// other is added.  Past them (at most rbq - 1 + 7 keys) a pair whose row ends
+// last are seen by every pair: they go 8 a chunk, three chunks in flight, through
+// buffer loads whose position is one scalar (354 -> 347 us at the 8B shape, 2048
+// rows, 32.0 -> 29.8 at 333 rows of hd 64, against one chunk in flight and a 64-bit
+// address per load; two and four chunks the same).  Past them (at most rbq - 1 + 7 keys) a pair whose row ends
 // before t supplies a zero weight, so its products are +-0 and its sums do not
 // move; should such a key's V value not be finite (0 * inf is NaN), that key
 // masks the products element by element instead.
@@ -1315,32 +1381,36 @@ __global__ __launch_bounds__(64 * (32 / NP) * ((HD + 63) / 64)) __attribute__((a
     s += S::outer(a, b);
     __builtin_amdgcn_sched_barrier(0);                               // one product tile live at a time
   };
-  if (k8 > 0) {
-    float4 xa0 = *reinterpret_cast<const float4 *>(wr), xa1 = *reinterpret_cast<const float4 *>(wr + 4);
-    float xb[8], yb[8];
-    float4 ya0, ya1;
+  constexpr int D = 3;                                               // chunks in flight
+  const __amdgpu_buffer_rsrc_t rw = mx_rsrc(w + (size_t)kvh * G * R * Tp, G * R * Tp);
+  const __amdgpu_buffer_rsrc_t rv = mx_rsrc(vc + (size_t)kvh * max_seq * HD, max_seq * HD);
+  const int ow = (ga * R + ra) * Tp * 4, ov = min(d0 + lane, HD - 1) * 4;
+  float4 xa[D][2];
+  float xb[D][8];
+  auto load = [&](int d, int t) __attribute__((always_inline)) {     // keys t .. t+7 (past the last: read, not added)
+    xa[d][0] = mx_load16(rw, ow, t * 4);
+    xa[d][1] = mx_load16(rw, ow + 16, t * 4);
 #pragma unroll
-    for (int u = 0; u < 8; u++) xb[u] = vr[u * HD];
-    for (int t = 0; t < k8; t += 16) {
-      const int ty = min(t + 8, k8 - 8);
-      ya0 = *reinterpret_cast<const float4 *>(wr + ty);
-      ya1 = *reinterpret_cast<const float4 *>(wr + ty + 4);
+    for (int u = 0; u < 8; u++) xb[d][u] = mx_load4(rv, ov + u * HD * 4, t * HD * 4);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto sum = [&](int d) __attribute__((always_inline)) {
+    add(xa[d][0].x, xb[d][0]); add(xa[d][0].y, xb[d][1]); add(xa[d][0].z, xb[d][2]); add(xa[d][0].w, xb[d][3]);
+    add(xa[d][1].x, xb[d][4]); add(xa[d][1].y, xb[d][5]); add(xa[d][1].z, xb[d][6]); add(xa[d][1].w, xb[d][7]);
+  };
 #pragma unroll
-      for (int u = 0; u < 8; u++) yb[u] = vr[(size_t)(ty + u) * HD];
-      __builtin_amdgcn_sched_barrier(0);                             // the requests go out before the adds
-      add(xa0.x, xb[0]); add(xa0.y, xb[1]); add(xa0.z, xb[2]); add(xa0.w, xb[3]);
-      add(xa1.x, xb[4]); add(xa1.y, xb[5]); add(xa1.z, xb[6]); add(xa1.w, xb[7]);
-      if (t + 8 >= k8) break;
-      const int tx = min(t + 16, k8 - 8);
-      xa0 = *reinterpret_cast<const float4 *>(wr + tx);
-      xa1 = *reinterpret_cast<const float4 *>(wr + tx + 4);
+  for (int d = 0; d < D; d++) load(d, 8 * d);
+  int t = 0;
+  for (; t + 8 * D <= k8; t += 8 * D) {
 #pragma unroll
-      for (int u = 0; u < 8; u++) xb[u] = vr[(size_t)(tx + u) * HD];
-      __builtin_amdgcn_sched_barrier(0);
-      add(ya0.x, yb[0]); add(ya0.y, yb[1]); add(ya0.z, yb[2]); add(ya0.w, yb[3]);
-      add(ya1.x, yb[4]); add(ya1.y, yb[5]); add(ya1.z, yb[6]); add(ya1.w, yb[7]);
+    for (int d = 0; d < D; d++) {
+      sum(d);
+      load(d, t + 8 * (d + D));
     }
   }
+#pragma unroll
+  for (int d = 0; d < D - 1; d++)
+    if (t + 8 * d < k8) sum(d);
   // the rest (past the first row's last key the keys are masked per pair), 8
   // keys a batch: a pair whose row ends before a key supplies a zero weight, and
   // past the last key the V value is zero too; a batch with a masked key whose

@@ -232,6 +232,28 @@ def test_batched_prefill_groupings_match_oracle(Q, shape, path):
         ref.close()
 
 
+@pytest.mark.parametrize("shape", [(10, 2, 64, 1), (12, 2, 48, 63), (7, 1, 128, 65), (5, 1, 64, 129), (6, 1, 48, 258)],
+                         ids=lambda s: f"G{s[0] // s[1]}hd{s[2]}n{s[3]}")
+def test_prompt_attention_block_edges_match_oracle(Q, shape):
+    """Prompt attention where its pair and key blocks end: groups of 5, 6 and 7
+    query heads (32 pairs hold idle ones), prompts around one wave's 64 keys and
+    one block's 256, then a second piece behind them: every logit vector and the
+    steps after, bit for bit against the oracle."""
+    H, KVH, hd, n = shape
+    cfg = [300, 320, 1, H, KVH, hd, 384, n + 40]
+    ids = O.prompt(n + 19, 5, cfg[0])
+    ref, m = O.Model(cfg, 10000.0, seed=n), Q.Model.synth(cfg, 10000.0, seed=n)
+    try:
+        for lo, hi in ((0, n), (n, n + 19)):
+            for t in ids[lo:hi]:
+                ref.step(t)
+            assert bits_equal(m.prefill(ids[lo:hi]), ref.logits)
+        assert bits_equal(m.step(7), ref.step(7))
+    finally:
+        m.close()
+        ref.close()
+
+
 def test_decode_rejects_position_past_max_seq(Q):
     # the reference leaves this to its callers (main.c:663); the library checks
     # it on the host before any device work: run in a child so the abort is seen
