@@ -538,6 +538,85 @@ __global__ __launch_bounds__(256) void k_gemv_dec_any(const int8_t *qa, const fl
   }
 }
 
+// Short rows (kpad <= 1024: a lane's 16 bytes are its whole share of a row): the
+// block forms its quantized activation itself, from v's rmsnorm (PRO 2, the
+// operations of k_rmsnorm_quant) or from v and its producer's block maxima (PRO 1,
+// k_quant_blocks), one word a thread into LDS, while the four rows' weights are in
+// flight.  A wave then is one row.
+// Bound: latency, of the prologue's reductions and of the launch; the separate
+// kernel before it cost as much and a boundary more.  Kernel times before and after
+// at kpad 288: rmsnorm + QKV 5.0 + 2.8 -> 4.5 us, rmsnorm + gate|up 5.0 + 3.1 -> 5.0,
+// quantization + Wo or down (kpad 768) 1.8 + 2.8 -> 2.8.
+template <int MODE, int PRO>
+__global__ __launch_bounds__(256) void k_gemv_small(const float *v, int n, const float *g, int nvbm, float eps,
+                                                    const int8_t *W, const float *ws, int N, int kpad, float *out,
+                                                    const float *bias, float *bm) {
+  constexpr bool U = MODE == MODE_SWIGLU;
+  __shared__ __attribute__((aligned(16))) uint32_t qs[256];
+  __shared__ float red[4];
+  __shared__ qd::SeqScratch seq;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int j = blockIdx.x * 4 + wave, jc = min(j, N - 1);
+  float y[4], gm[4], mx = 0.0f;
+  if constexpr (PRO == 2) {
+    qd::rmsnorm_load<4>(v, n, g, y, gm);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) y[i] = 4 * t + i < n ? v[4 * t + i] : 0.0f;
+    for (int i = t; i < nvbm; i += 256) mx = fmaxf(mx, g[i]);
+  }
+  __builtin_amdgcn_sched_barrier(0);          // the row first: loads return in order
+  const int lc = min(lane, (kpad >> 4) - 1);
+  const int4 wv = reinterpret_cast<const int4 *>(W + (size_t)jc * kpad)[lc];
+  const int4 uv = U ? reinterpret_cast<const int4 *>(W + (size_t)(N + jc) * kpad)[lc] : int4{};
+  const float wsj = ws[jc], wsu = U ? ws[N + jc] : 0.0f;
+  const float add = MODE == MODE_RESID ? out[jc] : MODE == MODE_PLAIN && bias ? bias[jc] : 0.0f;
+  __builtin_amdgcn_sched_barrier(0);
+  float as;
+  if constexpr (PRO == 2) {
+    as = qd::rmsnorm_apply<256, 4>(v, n, eps, y, gm, red, seq);
+  } else {
+    mx = qd::wave_max_f32(mx);
+    if (lane == 0) red[wave] = mx;
+    qd::lds_sync();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    as = (mx > 0.0f) ? mx / 127.0f : 1.0f;
+  }
+  qs[t] = qd::quant_i8x4(y[0], y[1], y[2], y[3], 1.0f / as);     // 0 past n
+  qd::lds_sync();
+  int tw = 0, tu = 0;
+  if (lane < kpad >> 4) {
+    const int4 av = *reinterpret_cast<const int4 *>(&qs[4 * lane]);
+    tw = __builtin_amdgcn_sdot4(av.x, wv.x, tw, false);
+    tw = __builtin_amdgcn_sdot4(av.y, wv.y, tw, false);
+    tw = __builtin_amdgcn_sdot4(av.z, wv.z, tw, false);
+    tw = __builtin_amdgcn_sdot4(av.w, wv.w, tw, false);
+    if (U) {
+      tu = __builtin_amdgcn_sdot4(av.x, uv.x, tu, false);
+      tu = __builtin_amdgcn_sdot4(av.y, uv.y, tu, false);
+      tu = __builtin_amdgcn_sdot4(av.z, uv.z, tu, false);
+      tu = __builtin_amdgcn_sdot4(av.w, uv.w, tu, false);
+    }
+  }
+  const int sw = qd::wave_sum_i32(tw);
+  if (U) {
+    const int su = qd::wave_sum_i32(tu);
+    const float gt = (as * wsj) * (float)sw;
+    const float up = (as * wsu) * (float)su;
+    const float sg = 1.0f / (1.0f + qd::expf_glibc(-gt));
+    const float h = (gt * sg) * up;
+    if (lane == 0) {
+      if (j < N) out[j] = h;
+      red[wave] = j < N ? fabsf(h) : 0.0f;                       // the norm's maxima were read before the last barrier
+    }
+    qd::lds_sync();
+    if (t == 0) bm[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  } else if (lane == 0 && j < N) {
+    const float c = (as * wsj) * (float)sw;
+    out[j] = MODE == MODE_RESID ? add + c : bias ? c + add : c;
+  }
+}
+
 // Reduce the per-block (max, first index) candidates of the head GEMV to the
 // greedy token; then record it and advance the position (see qhip.h).
 __global__ __launch_bounds__(1024) void k_argmax_final(const float *bv, const int *bidx, int nb, int *d_in,
@@ -1174,6 +1253,32 @@ extern "C" int qhip_gemv_plain_norm(int cls, int fast, const float *x, int dm, c
 
 // Shapes qhip_gemv_resid_q supports.
 extern "C" int qhip_gemv_fused_ok(int kpad) { return kpad == 2048 || kpad == 4096 || kpad == 8192 || kpad == 14336; }
+
+// Shapes qhip_gemv_small takes: rows of one 16-byte word a lane, and no more blocks
+// than are resident together (four a CU), so that forming the activation in every
+// one of them costs no more than forming it once.
+extern "C" int qhip_gemv_small_ok(int N, int kpad) {
+  return N > 0 && kpad > 0 && kpad % 16 == 0 && kpad <= 1024 && (N + 3) / 4 <= 1024;
+}
+
+extern "C" int qhip_gemv_small(int mode, int cls, const float *v, int n, const float *g, int nvbm, float eps,
+                               const int8_t *W, const float *ws, int N, int kpad, float *out, const float *bias,
+                               float *bm) {
+  if (!qhip_gemv_small_ok(N, kpad) || n <= 0 || n > kpad) return qh::fail_msg("gemv_small: unsupported shape");
+  const dim3 grid((N + 3) / 4), block(256);
+  switch (mode) {
+    case MODE_PLAIN:
+      QH_LAUNCH(cls, (k_gemv_small<MODE_PLAIN, 2>), grid, block, 0, v, n, g, 0, eps, W, ws, N, kpad, out, bias, bm);
+      return 0;
+    case MODE_RESID:
+      QH_LAUNCH(cls, (k_gemv_small<MODE_RESID, 1>), grid, block, 0, v, n, g, nvbm, eps, W, ws, N, kpad, out, bias, bm);
+      return 0;
+    case MODE_SWIGLU:
+      QH_LAUNCH(cls, (k_gemv_small<MODE_SWIGLU, 2>), grid, block, 0, v, n, g, 0, eps, W, ws, N, kpad, out, bias, bm);
+      return 0;
+    default: return qh::fail_msg("gemv_small: bad mode");
+  }
+}
 
 extern "C" int qhip_quant_blocks(const float *v, int n, const float *bm, int nbm, int8_t *qa, int kpad, float *as) {
   QH_LAUNCH(QK_QUANT, k_quant_blocks, dim3((kpad + 1023) / 1024), dim3(256), 0, v, n, bm, nbm, qa, kpad, as);

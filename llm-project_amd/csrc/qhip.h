@@ -183,6 +183,12 @@ int qhip_gemv_norm_ok(int kpad, int dm);
 int qhip_gemv_plain_norm(int cls, int fast, const float *x, int dm, const float *gamma, float eps, const int8_t *W,
                          const float *ws, int N, int kpad, float *out, const float *bias);
 int qhip_gemv_norm_blocks(int N);
+// Short rows (qhip_gemv_small_ok): mode 0 (QKV) and 2 (gate|up, qhip_gemv_blocks
+// maxima) over rmsnorm(v) with gamma g, mode 1 (residual) over v quantized from
+// its producer's maxima g[nvbm]; the activation is formed inside.
+int qhip_gemv_small_ok(int N, int kpad);
+int qhip_gemv_small(int mode, int cls, const float *v, int n, const float *g, int nvbm, float eps, const int8_t *W,
+                    const float *ws, int N, int kpad, float *out, const float *bias, float *bm);
 // Quantize v (n values) into qa (kpad, zero padded) and *as from nbm per-block maxima.
 int qhip_quant_blocks(const float *v, int n, const float *bm, int nbm, int8_t *qa, int kpad, float *as);
 

@@ -680,6 +680,9 @@ static int enqueue_step(const QDev *d, const KVDev *kd) {
     } else if (fuse_gu) {       // rmsnorm inside the QKV GEMV
       rc |= qhip_gemv_plain_norm(2, fast, d->x, d->dm, d->g_attn[l], d->eps, d->wqkv[l], d->sqkv[l], d->nqkv,
                                  d->kp_dm, d->qkv, d->bqkv[l]);
+    } else if (qhip_gemv_small_ok(d->nqkv, d->kp_dm)) {
+      rc |= qhip_gemv_small(0, 2, d->x, d->dm, d->g_attn[l], 0, d->eps, d->wqkv[l], d->sqkv[l], d->nqkv, d->kp_dm,
+                            d->qkv, d->bqkv[l], NULL);
     } else {
       rc |= qhip_rmsnorm_quant(d->x, 1, d->dm, d->g_attn[l], d->eps, d->qa, d->kp_dm, d->as);
       rc |= qhip_gemv_dec(0, 2, d->qa, d->as, d->wqkv[l], d->sqkv[l], d->nqkv, d->kp_dm, d->qkv, d->bqkv[l], NULL, NULL);
@@ -692,6 +695,8 @@ static int enqueue_step(const QDev *d, const KVDev *kd) {
                                 d->rope_sin, d->scores, d->o, d->obm);
     if (fuse_o) {        // o quantized inside the Wo GEMV
       rc |= qhip_gemv_resid_q(6, d->o, d->qd, d->obm, nbo, d->wo[l], d->so[l], d->dm, d->kp_qd, d->x);
+    } else if (qhip_gemv_small_ok(d->dm, d->kp_qd)) {
+      rc |= qhip_gemv_small(1, 6, d->o, d->qd, d->obm, nbo, 0.0f, d->wo[l], d->so[l], d->dm, d->kp_qd, d->x, NULL, NULL);
     } else {
       rc |= qhip_quant_blocks(d->o, d->qd, d->obm, nbo, d->qa, d->kp_qd, d->as);
       rc |= qhip_gemv_dec(1, 6, d->qa, d->as, d->wo[l], d->so[l], d->dm, d->kp_qd, d->x, NULL, NULL, NULL);
@@ -699,6 +704,9 @@ static int enqueue_step(const QDev *d, const KVDev *kd) {
     if (fuse_gu) {       // rmsnorm inside the gate|up GEMV
       rc |= qhip_gemv_swiglu_norm(7, fast, d->x, d->dm, d->g_ffn[l], d->eps, d->wgu[l], d->sgu[l], d->dff, d->kp_dm,
                                   d->gu, d->hbm);
+    } else if (qhip_gemv_small_ok(d->dff, d->kp_dm)) {
+      rc |= qhip_gemv_small(2, 7, d->x, d->dm, d->g_ffn[l], 0, d->eps, d->wgu[l], d->sgu[l], d->dff, d->kp_dm, d->gu,
+                            NULL, d->hbm);
     } else {
       rc |= qhip_rmsnorm_quant(d->x, 1, d->dm, d->g_ffn[l], d->eps, d->qa, d->kp_dm, d->as);
       rc |= qhip_gemv_dec(2, 7, d->qa, d->as, d->wgu[l], d->sgu[l], d->dff, d->kp_dm, d->gu, NULL, d->hbm, NULL);
@@ -711,6 +719,9 @@ static int enqueue_step(const QDev *d, const KVDev *kd) {
     // more than the boundary it saves).
     if (d->kp_ff <= 8192 && qhip_gemv_fused_ok(d->kp_ff)) {
       rc |= qhip_gemv_resid_q(9, d->gu, d->dff, d->hbm, nbh, d->wd[l], d->sd[l], d->dm, d->kp_ff, d->x);
+    } else if (qhip_gemv_small_ok(d->dm, d->kp_ff)) {
+      rc |= qhip_gemv_small(1, 9, d->gu, d->dff, d->hbm, nbh, 0.0f, d->wd[l], d->sd[l], d->dm, d->kp_ff, d->x, NULL,
+                            NULL);
     } else {
       rc |= qhip_quant_blocks(d->gu, d->dff, d->hbm, nbh, d->qa, d->kp_ff, d->as);
       rc |= qhip_gemv_dec(1, 9, d->qa, d->as, d->wd[l], d->sd[l], d->dm, d->kp_ff, d->x, NULL, NULL, NULL);

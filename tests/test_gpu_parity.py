@@ -254,6 +254,23 @@ def test_prompt_attention_block_edges_match_oracle(Q, shape):
         ref.close()
 
 
+@pytest.mark.parametrize("dm,H,KVH,hd,dff", [(2, 1, 1, 2, 3), (1021, 4, 2, 48, 1009), (1024, 8, 2, 128, 1024),
+                                              (1025, 16, 4, 64, 1025), (64, 2, 1, 64, 4096), (64, 2, 2, 32, 4097),
+                                              (300, 17, 17, 60, 100)])
+def test_small_decode_gemv_edges_match_oracle(Q, dm, H, KVH, hd, dff):
+    """Decode steps of models whose GEMVs form their activation themselves, around
+    the longest row (1024) and the most blocks (4096 outputs) of that route, each
+    GEMV on its own side of the line: bit for bit against the oracle."""
+    cfg = [300, dm, 2, H, KVH, hd, dff, 32]
+    ref, m = O.Model(cfg, 10000.0, seed=dm), Q.Model.synth(cfg, 10000.0, seed=dm)
+    try:
+        for t in [3, 299, 0, 41]:
+            assert bits_equal(m.step(t), ref.step(t)), (cfg, t)
+    finally:
+        m.close()
+        ref.close()
+
+
 def test_decode_rejects_position_past_max_seq(Q):
     # the reference leaves this to its callers (main.c:663); the library checks
     # it on the host before any device work: run in a child so the abort is seen
