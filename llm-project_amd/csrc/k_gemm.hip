@@ -231,7 +231,8 @@ struct EpiLane {
   float w[2], b[2];
 };
 
-// All threads; published by the first barrier of the K loop.
+// All threads; epi_publish() before the K loop's first barrier makes the LDS part
+// readable by the block's other waves behind it.
 template <int MODE, int TM, int NT>
 __device__ __forceinline__ EpiLane<MODE> epi_begin(EpiShared<TM> &sh, const float *as, const float *ws,
                                                    const float *bias, int M, int N, int m0, int n0, int wn, int lane) {
@@ -253,6 +254,11 @@ __device__ __forceinline__ EpiLane<MODE> epi_begin(EpiShared<TM> &sh, const floa
   }
   return l;
 }
+
+// The K loop's barriers are bare (no fence): a wave's LDS writes of epi_begin have to
+// have landed when it reaches the first one, or after a single K step another wave's
+// epilogue may read before them.  One wait a block, behind the first copies' requests.
+__device__ __forceinline__ void epi_publish() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // The wave's sums to the output: result element e of row block a is row i0 + 32 a +
 // 8 (e / 4) + 4 (lane / 32) + e % 4, i0 = r0 rows into the block's m0.  FULL: every
@@ -489,6 +495,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_i8_pipe(const int8_t *A, 
   issue(std::integral_constant<int, 0>(), 0);
   if (1 < nk) issue(std::integral_constant<int, 1>(), 1);
   if (NSTAGE > 3 && 2 < nk) issue(std::integral_constant<int, (NSTAGE > 3 ? 2 : 0)>(), 2);
+  epi_publish();
   for (int kt = 0; kt < nk; kt += NSTAGE) {
     step(std::integral_constant<int, 0>(), kt);
     if (kt + 1 < nk) step(std::integral_constant<int, 1>(), kt + 1);
@@ -712,6 +719,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
   for (int i = 0; i < NS; i++)
     if (i < nk) issue(i, i);
+  epi_publish();
   if (nk >= NS) wait_vmcnt<LPS * (NS - 1)>();
   else wait_vmcnt<0>();
   block_sync_lds();
