@@ -78,10 +78,11 @@ __device__ __forceinline__ void f_sum(float &acc, const float4 &p, Mid mid) {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// 16 bytes of a buffer resource at the lane's offset vo plus the wave's so (bytes);
-// 0 past the resource's end.
-__device__ __forceinline__ float4 f_load16(__amdgpu_buffer_rsrc_t rs, int vo, int so) {
-  const auto r = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0);
+// 16 bytes of a buffer resource at the lane's offset vo (bytes); 0, and no memory
+// traffic, past the resource's end.  The whole offset is in the vector operand: the
+// range check does not cover the scalar one.
+__device__ __forceinline__ float4 f_load16(__amdgpu_buffer_rsrc_t rs, int vo) {
+  const auto r = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, 0, 0);
   float4 v;
   __builtin_memcpy(&v, &r, 16);
   return v;
@@ -110,14 +111,22 @@ __global__ __launch_bounds__(64) void k_gemv_f32(const float *x, int K, const fl
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, K * 4, 0x00020000);
   const int vw = lane * 16, vx = (16 * c + 4 * s) * 4;
   float4 w[kFD][4], xv[kFD];
-  auto loadw = [&](int d, int g, int t) { w[d][t] = f_load16(rw, vw + t * kFTile * 4, g * 4 * kFTile * 4); };
-  auto loadx = [&](int d, int g) { xv[d] = f_load16(rx, vx, g * 4 * kFK * 4); };   // past the last group: reads 0, no traffic
+  // the offsets of the group to request next: one register each, the tile a constant beside it
+  int ow = vw, ox = vx;
+  auto loadw = [&](int d, int t) __attribute__((always_inline)) { w[d][t] = f_load16(rw, ow + t * kFTile * 4); };
+  auto loadx = [&](int d) __attribute__((always_inline)) { xv[d] = f_load16(rx, ox); };
+  auto next = [&]() __attribute__((always_inline)) {
+    ow += 4 * kFTile * 4;
+    ox += 4 * kFK * 4;
+    asm volatile("" : "+v"(ow), "+v"(ox));
+  };
   float acc = 0.0f;
 #pragma unroll
   for (int d = 0; d < kFD; d++) {
 #pragma unroll
-    for (int t = 0; t < 4; t++) loadw(d, d, t);
-    loadx(d, d);
+    for (int t = 0; t < 4; t++) loadw(d, t);
+    loadx(d);
+    next();
     __builtin_amdgcn_sched_barrier(0);      // groups arrive in order: a wait for one leaves the later ones in flight
   }
   int g0 = 0;
@@ -127,7 +136,7 @@ __global__ __launch_bounds__(64) void k_gemv_f32(const float *x, int K, const fl
   for (; g0 + kFD < ng; g0 += kFD) {        // whole rounds: no branch inside, so the waits name only the loads in use
 #pragma unroll
     for (int d = 0; d < kFD; d++) {
-      const int g = g0 + d + kFD, e = (d + 1) % kFD;
+      const int e = (d + 1) % kFD;
       float4 q;
       f_sum(acc, p, [&](int i) {
         if (i == 0) q.x = f_dpp<0x55>(xv[d].x) * w[d][1].x;
@@ -136,23 +145,26 @@ __global__ __launch_bounds__(64) void k_gemv_f32(const float *x, int K, const fl
         if (i == 3) q.w = f_dpp<0x55>(xv[d].w) * w[d][1].w;
       });
       f_sum(acc, q, [&](int i) {
-        if (i == 1) loadw(d, g, 0);
+        if (i == 1) loadw(d, 0);
         if (i == 0) p.x = f_dpp<0xaa>(xv[d].x) * w[d][2].x;
         if (i == 1) p.y = f_dpp<0xaa>(xv[d].y) * w[d][2].y;
         if (i == 2) p.z = f_dpp<0xaa>(xv[d].z) * w[d][2].z;
         if (i == 3) p.w = f_dpp<0xaa>(xv[d].w) * w[d][2].w;
       });
       f_sum(acc, p, [&](int i) {
-        if (i == 1) loadw(d, g, 1);
+        if (i == 1) loadw(d, 1);
         if (i == 0) q.x = f_dpp<0xff>(xv[d].x) * w[d][3].x;
         if (i == 1) q.y = f_dpp<0xff>(xv[d].y) * w[d][3].y;
         if (i == 2) q.z = f_dpp<0xff>(xv[d].z) * w[d][3].z;
         if (i == 3) q.w = f_dpp<0xff>(xv[d].w) * w[d][3].w;
       });
       f_sum(acc, q, [&](int i) {
-        if (i == 1) loadw(d, g, 2);
-        if (i == 2) loadw(d, g, 3);
-        if (i == 3) loadx(d, g);
+        if (i == 1) loadw(d, 2);
+        if (i == 2) loadw(d, 3);
+        if (i == 3) {
+          loadx(d);
+          next();
+        }
         if (i == 0) p.x = f_dpp<0>(xv[e].x) * w[e][0].x;
         if (i == 1) p.y = f_dpp<0>(xv[e].y) * w[e][0].y;
         if (i == 2) p.z = f_dpp<0>(xv[e].z) * w[e][0].z;
@@ -174,7 +186,7 @@ __global__ __launch_bounds__(64) void k_gemv_f32(const float *x, int K, const fl
     const int k0 = ng * 4 * kFK + 16 * c + 4 * s;
     float4 wt[4], xt;
 #pragma unroll
-    for (int t = 0; t < 4; t++) wt[t] = f_load16(rw, vw + t * kFTile * 4, 4 * ng * kFTile * 4);
+    for (int t = 0; t < 4; t++) wt[t] = f_load16(rw, vw + (4 * ng + t) * kFTile * 4);       // 0 past the panel
     xt.x = k0 < K ? x[k0] : 0.0f;
     xt.y = k0 + 1 < K ? x[k0 + 1] : 0.0f;
     xt.z = k0 + 2 < K ? x[k0 + 2] : 0.0f;
@@ -274,9 +286,14 @@ __global__ __launch_bounds__(64 * kFNW) void k_gemv_f32_norm(const float *x, int
   }
   const int vw = lane * 16;
   float4 w[kFD][NP][4], xv[kFD];
-  auto loadw = [&](int d, int g, int t) __attribute__((always_inline)) {       // past the panel's end: reads 0, no traffic
+  int ow = vw;                                // of the group to request next
+  auto loadw = [&](int d, int t) __attribute__((always_inline)) {       // past the panel's end: reads 0, no traffic
 #pragma unroll
-    for (int n = 0; n < NP; n++) w[d][n][t] = f_load16(rw[n], vw + t * kFTile * 4, g * 4 * kFTile * 4);
+    for (int n = 0; n < NP; n++) w[d][n][t] = f_load16(rw[n], ow + t * kFTile * 4);
+  };
+  auto next = [&]() __attribute__((always_inline)) {
+    ow += 4 * kFTile * 4;
+    asm volatile("" : "+v"(ow));
   };
   auto loadx = [&](int d, int g) __attribute__((always_inline)) {              // groups past the last: the last again
     xv[d] = *reinterpret_cast<const float4 *>(&xs[min(g, ng - 1) * 4 * kFK + 16 * c + 4 * s]);
@@ -284,7 +301,8 @@ __global__ __launch_bounds__(64 * kFNW) void k_gemv_f32_norm(const float *x, int
 #pragma unroll
   for (int d = 0; d < kFD; d++) {
 #pragma unroll
-    for (int t = 0; t < 4; t++) loadw(d, d, t);
+    for (int t = 0; t < 4; t++) loadw(d, t);
+    next();
     __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (PRO == FPRO_LN) qd::layernorm_apply<NT, CM>(x, K, eps, y, gm, be, xs, &red[0], seq);
@@ -336,12 +354,15 @@ __global__ __launch_bounds__(64 * kFNW) void k_gemv_f32_norm(const float *x, int
     for (int d = 0; d < kFD; d++) {
       const int g = g0 + d + kFD, e = (d + 1) % kFD;
       tile(C1(), p[0], p[1], w[d], xv[d], none);
-      tile(C2(), p[1], p[0], w[d], xv[d], [&](int i) __attribute__((always_inline)) { if (i == 1) loadw(d, g, 0); });
-      tile(C3(), p[0], p[1], w[d], xv[d], [&](int i) __attribute__((always_inline)) { if (i == 1) loadw(d, g, 1); });
+      tile(C2(), p[1], p[0], w[d], xv[d], [&](int i) __attribute__((always_inline)) { if (i == 1) loadw(d, 0); });
+      tile(C3(), p[0], p[1], w[d], xv[d], [&](int i) __attribute__((always_inline)) { if (i == 1) loadw(d, 1); });
       tile(C0(), p[1], p[0], w[e], xv[e], [&](int i) __attribute__((always_inline)) {
-        if (i == 1) loadw(d, g, 2);
-        if (i == 2) loadw(d, g, 3);
-        if (i == 3) loadx(d, g);
+        if (i == 1) loadw(d, 2);
+        if (i == 2) loadw(d, 3);
+        if (i == 3) {
+          loadx(d, g);
+          next();
+        }
       });
     }
   }

@@ -101,6 +101,61 @@ def test_f32_norm_in_gemv_edges_match_oracle(Q, dm, dff):
         ref.close()
 
 
+@pytest.mark.parametrize("K", [1, 17, 48, 80, 200, 288, 513, 768, 1040, 2000])
+@pytest.mark.parametrize("pro,mode", [(0, 0), (1, 0), (1, 4), (2, 3)])
+def test_f32_gemv_sees_its_own_panels_only(Q, pro, mode, K):
+    """Inputs that end inside a group of four tiles, or whose groups are fewer than
+    those in flight: with every second 16-column panel of the weights infinite, the
+    other panels' outputs are finite and, bit for bit, what they are with finite
+    neighbours (pro 0 plain, 1 rmsnorm, 2 LayerNorm; mode 4 SwiGLU, 3 GELU)."""
+    import ctypes as C
+    lib, N = Q.lib(), 64
+    cols = 2 * N if mode == 4 else N
+    lib.qllama_dev_alloc.restype = C.c_void_p
+    lib.qhip_panels_f32_size.restype = C.c_size_t
+    lib.qllama_dev_free.argtypes = [C.c_void_p]
+    lib.qllama_h2d.argtypes = lib.qllama_d2h.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t]
+    lib.qhip_to_panels_f32.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p]
+    lib.qhip_gemv_f32.argtypes = [C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]
+    lib.qhip_gemv_f32_norm.argtypes = [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_float,
+                                       C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+                                       C.c_int, C.c_int]
+    bufs = []
+
+    def dev(a):
+        p = lib.qllama_dev_alloc(C.c_size_t(a.nbytes))
+        assert p and lib.qllama_h2d(p, a.ctypes.data, a.nbytes) == 0
+        bufs.append(p)
+        return p
+
+    rng = np.random.default_rng(K)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    W = f(K, cols)
+    Winf = W.copy()
+    Winf[:, (np.arange(cols) // 16) % 2 == 1] = np.inf
+    try:
+        x, gamma, beta, bias = dev(f(K)), dev(f(K)), dev(f(K)), dev(f(N))
+        got = []
+        for w in (W, Winf):
+            panels = dev(np.zeros(lib.qhip_panels_f32_size(K, cols), np.float32))
+            out, dst = np.empty(N, np.float32), dev(np.zeros(N, np.float32))
+            assert lib.qhip_to_panels_f32(dev(w), K, cols, panels) == 0
+            if pro == 0:
+                assert lib.qhip_gemv_f32(mode, 12, x, K, panels, N, dst, bias) == 0
+            else:
+                assert lib.qhip_gemv_f32_norm(pro, mode, 12, x, K, gamma, beta, 1e-5, panels, N, dst,
+                                              None if mode == 4 else bias, None, None, None, 0, 0) == 0
+            assert lib.qllama_d2h(out.ctypes.data, dst, out.nbytes) == 0
+            got.append(out)
+    finally:
+        lib.qllama_sync()
+        for p in bufs:
+            lib.qllama_dev_free(p)
+    own = (np.arange(N) // 16) % 2 == 0
+    assert np.isfinite(got[1][own]).all()
+    assert np.array_equal(bits(got[0][own]), bits(got[1][own]))
+
+
 @pytest.mark.parametrize("rows,dff,vocab", [(1, 33, 70), (5, 64, 17), (9, 100, 130), (40, 31, 64), (70, 95, 2100),
                                             (300, 66, 16384)])
 def test_f32_forward_tile_edges_match_oracle(Q, rows, dff, vocab):
