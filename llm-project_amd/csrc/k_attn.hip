@@ -1227,18 +1227,22 @@ template <> struct MxShape<16> {
   __device__ static int col(int r, int l) { return 16 * (r >> 2) + (l & 15); }
 };
 
-// Buffer accesses of `n` floats from base: a byte offset a lane, one per wave, and
-// the range check (past n: reads 0, stores nothing).
+// Buffer accesses of `n` floats from base at a lane's byte offset, under the range
+// check (past n: reads 0, stores nothing, no memory traffic).  The whole offset is in
+// the vector operand, as in pv_load: the check does not cover the scalar one.
+// kMxPast is an offset past every buffer here (at most 1 GiB) that can still be
+// added to an offset inside it.
+constexpr int kMxPast = 0x40000000;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t mx_rsrc(const float *base, int n) {
   return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, n * 4, 0x00020000);
 }
-__device__ __forceinline__ float4 mx_load16(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+__device__ __forceinline__ float4 mx_load16(__amdgpu_buffer_rsrc_t r, int off) {
   typedef unsigned v4u __attribute__((ext_vector_type(4)));
-  const v4u t = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
+  const v4u t = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
   return make_float4(__uint_as_float(t.x), __uint_as_float(t.y), __uint_as_float(t.z), __uint_as_float(t.w));
 }
-__device__ __forceinline__ float mx_load4(__amdgpu_buffer_rsrc_t r, int off, int soff) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
+__device__ __forceinline__ float mx_load4(__amdgpu_buffer_rsrc_t r, int off) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
 __device__ __forceinline__ void mx_store4(__amdgpu_buffer_rsrc_t r, int off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0);
@@ -1276,8 +1280,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   static_assert(HD % 16 == 0, "whole halves of a line");
   float4 kb[2][4];
   auto kload = [&](auto bv, int h) __attribute__((always_inline)) {  // 64 bytes of the lane's key: dims 16h .. 16h+15
+    const int at = ok + (h < NH ? 64 * h : kMxPast);                 // past the row: nothing
 #pragma unroll
-    for (int i = 0; i < 4; i++) kb[decltype(bv)::value][i] = mx_load16(rk, ok + 16 * i, 64 * h);
+    for (int i = 0; i < 4; i++) kb[decltype(bv)::value][i] = mx_load16(rk, at + 16 * i);
   };
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
@@ -1319,7 +1324,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 #pragma unroll
       for (int i = 0; i < 4; i++) kb[0][i] = kb[1][i];
     }
-    kload(std::integral_constant<int, NH % 2 ? 1 : B>(), h + 2);     // past the row: the next key's, or 0; not added
+    kload(std::integral_constant<int, NH % 2 ? 1 : B>(), h + 2);
     __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll 1
@@ -1387,11 +1392,12 @@ __global__ __launch_bounds__(64 * (32 / NP) * ((HD + 63) / 64)) __attribute__((a
   const int ow = (ga * R + ra) * Tp * 4, ov = min(d0 + lane, HD - 1) * 4;
   float4 xa[D][2];
   float xb[D][8];
-  auto load = [&](int d, int t) __attribute__((always_inline)) {     // keys t .. t+7 (past the last: read, not added)
-    xa[d][0] = mx_load16(rw, ow, t * 4);
-    xa[d][1] = mx_load16(rw, ow + 16, t * 4);
+  auto load = [&](int d, int t) __attribute__((always_inline)) {     // keys t .. t+7; past the last chunk: nothing
+    const int aw = ow + (t < k8 ? t * 4 : kMxPast), av = ov + (t < k8 ? t * HD * 4 : kMxPast);
+    xa[d][0] = mx_load16(rw, aw);
+    xa[d][1] = mx_load16(rw, aw + 16);
 #pragma unroll
-    for (int u = 0; u < 8; u++) xb[d][u] = mx_load4(rv, ov + u * HD * 4, t * HD * 4);
+    for (int u = 0; u < 8; u++) xb[d][u] = mx_load4(rv, av + u * HD * 4);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto sum = [&](int d) __attribute__((always_inline)) {

@@ -9,7 +9,7 @@ import pytest
 
 import qlib
 
-FILES = ["k_gemv_f32.hip"]
+FILES = ["k_attn.hip", "k_fattn.hip", "k_gemv_f32.hip"]
 
 
 def arguments(text, at):

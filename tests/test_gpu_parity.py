@@ -254,6 +254,28 @@ def test_prompt_attention_block_edges_match_oracle(Q, shape):
         ref.close()
 
 
+@pytest.mark.parametrize("shape", [(6, 2, 48, 300), (8, 2, 64, 264), (16, 2, 64, 257), (8, 2, 128, 520),
+                                   (4, 1, 128, 2048)], ids=lambda s: f"H{s[0]}kv{s[1]}hd{s[2]}T{s[3]}")
+def test_prefill_to_the_last_cache_position_matches_oracle(Q, shape):
+    """A prompt that ends at the cache's last position, whole and behind a first
+    piece: prompt attention's requests ahead then lie past the last head's rows,
+    the end of the allocation for the last layer.  Bit for bit against the oracle."""
+    H, KVH, hd, n = shape
+    cfg = [300, 256, 2, H, KVH, hd, 256, n]
+    ids = O.prompt(n, 11, cfg[0])
+    ref, m = O.Model(cfg, 10000.0, seed=n), Q.Model.synth(cfg, 10000.0, seed=n)
+    try:
+        for t in ids:
+            ref.step(t)
+        assert bits_equal(m.prefill(ids), ref.logits)
+        m.reset(0)
+        m.prefill(ids[:n - 21], want_logits=False)
+        assert bits_equal(m.prefill(ids[n - 21:]), ref.logits)
+    finally:
+        m.close()
+        ref.close()
+
+
 @pytest.mark.parametrize("dm,H,KVH,hd,dff", [(2, 1, 1, 2, 3), (1021, 4, 2, 48, 1009), (1024, 8, 2, 128, 1024),
                                               (1025, 16, 4, 64, 1025), (64, 2, 1, 64, 4096), (64, 2, 2, 32, 4097),
                                               (300, 17, 17, 60, 100)])
