@@ -1257,10 +1257,8 @@ __device__ __forceinline__ void mx_store4(__amdgpu_buffer_rsrc_t r, int off, flo
 // (smaller steps would fetch a line from L2 once for each of them).
 // Bound: a SIMD's issue of MFMAs and adds, which do not overlap (64.5 ns per 2048
 // products: 264 us at the 8B shape, 2048 rows).  Held to 4 waves per SIMD (128
-// registers): the issue rate rises with a SIMD's waves.  383 -> 345 us at that
-// shape and 22.1 -> 19.2 at 333 rows of hd 64 against q and K both from memory a
-// line at a time and each element's address and test formed on its own (about 600
-// instructions a wave, many of them multiplies, after 4096 adds).
+// registers): the issue rate rises with a SIMD's waves.  356 us at that shape (332 on
+// a cool card, under a kernel trace) and 20.1 at 333 rows of hd 64.
 template <int HD, int NP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_pf_scores_mx(const float *q, const float *kc, int R, int p0, int H,
                                                       int KVH, int max_seq, float scale, float *w, int Tp) {

@@ -17,8 +17,8 @@
 //    of 128 bytes, v_mfma_i32_32x32x32_i8 (the 16x16x64 form runs at half its rate on
 //    gfx950).  Both operand tiles are copied straight from global memory into LDS
 //    (global_load_lds, no staging registers), two to four K steps in LDS.
-//  - k_gemm_i8_pipe (kpad % 64 == 0): 128 x 128 tiles, K steps of 64 bytes, 8 waves,
-//    four steps in LDS.
+//  - k_gemm_i8_pipe (kpad % 64 == 0): 128 x 128 or 256 x 128 tiles, K steps of 64
+//    bytes, 8 waves, four or three steps in LDS.
 //  - k_gemm_i8 (other K): 128 x 128 tiles staged through registers into
 //    double-buffered LDS, 4 waves of 4 x 4 v_mfma_i32_16x16x64_i8; chunks past
 //    kpad are zero.
@@ -231,8 +231,12 @@ struct EpiLane {
   float w[2], b[2];
 };
 
-// All threads; epi_publish() before the K loop's first barrier makes the LDS part
-// readable by the block's other waves behind it.
+// All threads.  The K loop's barriers are bare (no fence), so the LDS part is readable
+// by the block's other waves behind the first barrier that a wave reaches with its LDS
+// writes landed: k_gemm_i8_pipe waits for them before its first barrier (epi_publish;
+// after a single K step there is no other), k_gemm_i8_deep in the phase between its
+// first barrier and the loop's, whose wait is lgkmcnt(0) (a wait before the first one
+// as well cost 0.45 of 46.5 us at 1000 x 4096 x 6144).
 template <int MODE, int TM, int NT>
 __device__ __forceinline__ EpiLane<MODE> epi_begin(EpiShared<TM> &sh, const float *as, const float *ws,
                                                    const float *bias, int M, int N, int m0, int n0, int wn, int lane) {
@@ -255,9 +259,6 @@ __device__ __forceinline__ EpiLane<MODE> epi_begin(EpiShared<TM> &sh, const floa
   return l;
 }
 
-// The K loop's barriers are bare (no fence): a wave's LDS writes of epi_begin have to
-// have landed when it reaches the first one, or after a single K step another wave's
-// epilogue may read before them.  One wait a block, behind the first copies' requests.
 __device__ __forceinline__ void epi_publish() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // The wave's sums to the output: result element e of row block a is row i0 + 32 a +
@@ -560,7 +561,7 @@ int launch_pipe(const int8_t *A, const float *as, const int8_t *W, const float *
   const int blocks = 8 * mt * ((nt + 7) / 8);
   const int nkt = kpad / BK;
   int S = 1;
-  if (work) {
+  if (TM == 128 && work) {               // (the larger tile is taken only where it fills the CUs)
     const int cus = qh::num_cus() > 0 ? qh::num_cus() : 256, active = mt * nt;
     if (active < cus) {
       S = min(min((cus + active - 1) / active, nkt / 8), kMaxSplits);
@@ -574,13 +575,15 @@ int launch_pipe(const int8_t *A, const float *as, const int8_t *W, const float *
               N, kpad, out, ldo, bias, mt, nt, blocks, nkt, static_cast<int *>(nullptr));
     return 0;
   }
-  const int nks = (nkt + S - 1) / S;
-  S = (nkt + nks - 1) / nks;                                       // every split has steps
-  g_last_splits = S;
-  QH_LAUNCH(cls, (k_gemm_i8_pipe<MODE, TM, TN, WM, WN, NS, true>), dim3(blocks * S), dim3(64 * WM * WN), 0, A, as, W,
-            ws, M, N, kpad, out, ldo, bias, mt, nt, blocks, nks, work);
-  QH_LAUNCH(cls, k_gemm_split_epi<MODE>, dim3((N + 255) / 256, M), dim3(256), 0, work, S, as, ws, M, N, out, ldo,
-            bias);
+  if constexpr (TM == 128) {
+    const int nks = (nkt + S - 1) / S;
+    S = (nkt + nks - 1) / nks;                                     // every split has steps
+    g_last_splits = S;
+    QH_LAUNCH(cls, (k_gemm_i8_pipe<MODE, TM, TN, WM, WN, NS, true>), dim3(blocks * S), dim3(64 * WM * WN), 0, A, as,
+              W, ws, M, N, kpad, out, ldo, bias, mt, nt, blocks, nks, work);
+    QH_LAUNCH(cls, k_gemm_split_epi<MODE>, dim3((N + 255) / 256, M), dim3(256), 0, work, S, as, ws, M, N, out, ldo,
+              bias);
+  }
   return 0;
 }
 
@@ -597,6 +600,12 @@ int launch_pipe(const int8_t *A, const float *as, const int8_t *W, const float *
 // barrier of a step sits before its last phase: every wave has then read all of the
 // step's fragments, so its buffer takes the copies of step + NS, and the copies of
 // the next step, issued NS - 1 steps ago, have landed for the reads of that phase.
+// Limit: the compiler's hazard recognizer does not see the products inside the asm
+// blocks.  They follow one another without gaps (a block reads the sums only as the
+// products' own accumulators, for which the hardware waits), and the s_nops behind the
+// loop cover the last ones; but nothing else may read or move the sums between two
+// blocks: no operation on acc there, and no spill or copy of it (the accumulators and
+// fragments fit: the build's resource report shows no scratch for these kernels).
 // ---------------------------------------------------------------------------
 constexpr int DK = 128;
 
@@ -719,7 +728,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
   for (int i = 0; i < NS; i++)
     if (i < nk) issue(i, i);
-  epi_publish();
   if (nk >= NS) wait_vmcnt<LPS * (NS - 1)>();
   else wait_vmcnt<0>();
   block_sync_lds();
@@ -729,7 +737,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
   for (int a = 0; a < RB; a++) ya[a] = (v4i){};
 #pragma unroll
   for (int b = 0; b < 2; b++) yb[b] = (v4i){};
-  gemm_phase<BOFF>(acc, ya, yb, xa, xb, la[0], lb[0]);
+  gemm_phase<BOFF>(acc, ya, yb, xa, xb, la[0], lb[0]);   // its wait also covers epi_begin's LDS writes
   int buf = 0;
   for (int kt = 0; kt < nk; kt++) {
     const unsigned o = buf * STAGE;
@@ -776,7 +784,7 @@ int launch_deep(const int8_t *A, const float *as, const int8_t *W, const float *
   return qh::fail_msg("gemm_i8: this tile does not split K");
 }
 
-// Tile choice for kpad % 128 == 0, by the time of each in tenths of a microsecond
+// Tile choice for kpad % 128 == 0, by the time of each in hundredths of a microsecond
 // (measured on 2048, 1500, 1000, 512, 333, 200, 100 and 40 rows of the 8B and 1B
 // layers' products): a round of blocks takes a fixed part (first copies, epilogue)
 // and a part a step of 128 bytes of K,
@@ -788,6 +796,13 @@ int launch_deep(const int8_t *A, const float *as, const int8_t *W, const float *
 // planes written and read at 3 TB/s).  At 2048 rows, us: 8B gate|up 276 317 313
 // (256 x 256, 256 x 128, 128 x 128), QKV 61 71 65, Wo 86 52 46, down 189 126 131; 1B
 // down at 333 rows unsplit 43, split 5 ways 22.
+// kpad % 128 == 64 (steps of 64 bytes): 128 x 128, 8 waves, or for residual and
+// SwiGLU, where its tiles fill the CUs and the rounds cost less, 256 x 128,
+//   128 x 128, four steps in LDS                       1.65 + 0.35 us a step and round
+//   256 x 128, three steps in LDS                      5.60 + 0.54
+// us, 128 x 128 and 256 x 128: SwiGLU 2048 x 11008, K 4160 257 234; 800 x 11008, K 4160
+// 117 123; 2048 x 4224, K 1600 51 56; 2048 x 5632, K 2112 78 72; residual 2048 x 4096,
+// K 8256 105 90; 1500 x 6144, K 8256 138 147.
 template <int MODE>
 int launch(const int8_t *A, const float *as, const int8_t *W, const float *ws, int M, int N, int kpad, float *out,
            int ldo, const float *bias, int cls, int *work, size_t work_bytes) {
@@ -822,8 +837,16 @@ int launch(const int8_t *A, const float *as, const int8_t *W, const float *ws, i
       default: return launch_deep<MODE, 128, 128, 2, 2, 4>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, S, work);
     }
   }
-  if (kpad % BK == 0)
+  if (kpad % BK == 0) {
+    if constexpr (MODE != GM_PLAIN) {
+      const int cus = qh::num_cus() > 0 ? qh::num_cus() : 256, st = kpad / BK;
+      const long long nt = (N + (MODE == GM_SWIGLU ? 63 : 127)) / (MODE == GM_SWIGLU ? 64 : 128);
+      const long long t1 = (M + 127) / 128 * nt, t2 = (M + 255) / 256 * nt;
+      if (t2 >= cus && (t2 + cus - 1) / cus * (560 + 54 * st) < (t1 + cus - 1) / cus * (165 + 35 * st))
+        return launch_pipe<MODE, 256, 128, 4, 2, 3>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, work, work_bytes);
+    }
     return launch_pipe<MODE, 128, 128, 4, 2, 4>(A, as, W, ws, M, N, kpad, out, ldo, bias, cls, work, work_bytes);
+  }
   const int nout = MODE == GM_SWIGLU ? BN / 2 : BN;
   const int mt = (M + BM - 1) / BM, nt = (N + nout - 1) / nout;
   const int blocks = 8 * mt * ((nt + 7) / 8);

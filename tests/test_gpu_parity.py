@@ -608,6 +608,8 @@ def test_split_k_gemm_same_bits(Q, mode, M, N, kpad, bias):
     (1, 1800, 3900, 9728, False),
     # K a multiple of 64 but not of 128
     (0, 200, 300, 192, True), (1, 140, 520, 576, False), (2, 70, 90, 320, False),
+    # ... 256 x 128 blocks, the last row and column tile cut
+    (1, 2040, 4090, 960, False), (2, 2000, 2040, 1088, False),
     # one K step of 64: the epilogue's inputs meet the waves at a single barrier
     (0, 300, 500, 64, True), (1, 129, 260, 64, False), (2, 140, 200, 64, False)])
 def test_gemm_tiles_match_exact_sums(Q, mode, M, N, kpad, bias):
