@@ -11,6 +11,7 @@
 
 #include <limits.h>
 #include <math.h>
+#include <stdatomic.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -948,14 +949,19 @@ int q_llama_generate_greedy(const QLlamaModel *m, LlamaKV *kv, int token, int n_
 // created for it uploads a device copy (looked up by the model's weight
 // pointers), which lives as long as a cache of it does.  Weights are read at
 // that point: host changes made afterwards are seen by caches created later.
-// Device layout: every matrix keeps the reference's (K, N) row-major order (the
-// GEMV reads a row's columns contiguously); Wq|Wk|Wv and Wgate|Wup are joined
-// column-wise into one matrix each, so one launch serves each pair.
+// Device layout: every matrix in panels of 16 columns (qhip_to_panels_f32), the
+// embedding row-major; Wq|Wk|Wv and Wgate|Wup are joined column-wise into one
+// matrix each, so one launch serves each pair.
 // ---------------------------------------------------------------------------
+typedef struct {
+  void *p;             // device memory
+  size_t bytes;
+} FwdWs;
+
 typedef struct FDev {
   const void *key_wte, *key_blocks;      // identity of the host model
   uint64_t gen;                          // identifies this device copy to the graphs of its caches
-  int refs;
+  atomic_int refs;
   int vocab, dm, L, H, KVH, hd, dff, max_seq, qd, kvd, nqkv;
   float eps, attn_scale;
   uint8_t *blob;
@@ -964,23 +970,50 @@ typedef struct FDev {
   float *x, *xn, *qkv, *o, *gu, *h, *logits, *scores;
   int *d_state, *d_in;
   float *h_logits;     // pinned staging of one row of logits
-  void *ws;            // the batched forward's workspace, grown to the longest call
-  size_t ws_bytes;
+  _Atomic(FwdWs *) ws; // a workspace of the batched forward that no call holds (fwd_take)
 } FDev;
 
 #define FDEV_MAX 16
 static FDev *g_fdev[FDEV_MAX];
-// The pinned staging the batched forward's logits come back through: one for the
-// process (two chunks of FWD_DL_CHUNK), made by the first forward and given back
-// with the last fp32 model.
+// What the batched forward keeps from call to call.  A call takes it (leaving NULL) and
+// gives it back when it ends, so calls that overlap, on one model or on several, each
+// have their own and the surplus is freed.
+//  - a workspace per model, of at most FWD_KEEP_BYTES (a longer call's is freed with the
+//    call); freed with the model's device copy.
+//  - the pinned staging its logits come back through (two chunks of FWD_DL_CHUNK), one
+//    for the process; freed with the last fp32 model.
+#define FWD_KEEP_BYTES ((size_t)256 << 20)
 #define FWD_DL_CHUNK ((size_t)8 << 20)
-static void *g_fwd_dl;
+static _Atomic(void *) g_fwd_dl;
+
+static void fwd_ws_free(FwdWs *w) {
+  if (!w) return;
+  qhip_free(w->p);
+  free(w);
+}
+
+static FwdWs *fwd_take(FDev *f, size_t bytes) {
+  FwdWs *w = atomic_exchange(&f->ws, NULL);
+  if (w && w->bytes >= bytes) return w;
+  fwd_ws_free(w);
+  w = (FwdWs*)calloc(1, sizeof *w);
+  if (!w) return NULL;
+  w->p = qhip_malloc(bytes);
+  w->bytes = bytes;
+  if (!w->p) { free(w); return NULL; }
+  return w;
+}
+
+static void fwd_give(FDev *f, FwdWs *w) {
+  if (w && w->bytes <= FWD_KEEP_BYTES) w = atomic_exchange(&f->ws, w);
+  fwd_ws_free(w);
+}
 
 static void fdev_free(FDev *f) {
   if (!f) return;
   qhip_free(f->blob);
   qhip_host_free(f->h_logits);
-  qhip_free(f->ws);
+  fwd_ws_free(atomic_exchange(&f->ws, NULL));
   free(f->wqkv); free(f->bqkv); free(f->wo); free(f->wgu); free(f->wd); free(f->g_attn); free(f->g_ffn);
   free(f);
 }
@@ -994,7 +1027,7 @@ static void fdev_release(FDev *f) {
   }
   qhip_sync();
   fdev_free(f);
-  if (!others) { qhip_dl_free(g_fwd_dl); g_fwd_dl = NULL; }
+  if (!others) qhip_dl_free(atomic_exchange(&g_fwd_dl, NULL));
 }
 
 static FDev *fdev_find(const LlamaModel *m) {
@@ -1233,15 +1266,15 @@ static int fwd_run(FDev *f, float rope_base, const int *ids, int n, float *logit
   if (f->dff > kmax) kmax = f->dff;
   const size_t o_pk = FTAKE(qhip_gemm_f32_pack(R, kmax));
 #undef FTAKE
-  if (f->ws_bytes < off) {
-    qhip_sync();
-    qhip_free(f->ws);
-    f->ws = qhip_malloc(off);
-    f->ws_bytes = f->ws ? off : 0;
+  FwdWs *held = fwd_take(f, off);
+  void *dl = atomic_exchange(&g_fwd_dl, NULL);
+  if (!dl) dl = qhip_dl_create(FWD_DL_CHUNK);
+  if (!held || !dl) {
+    fwd_give(f, held);
+    qhip_dl_free(dl);
+    return 1;
   }
-  if (!g_fwd_dl) g_fwd_dl = qhip_dl_create(FWD_DL_CHUNK);
-  uint8_t *b = (uint8_t*)f->ws;
-  if (!b || !g_fwd_dl) return 1;
+  uint8_t *b = (uint8_t*)held->p;
   int *d_ids = (int*)(b + o_ids);
   float *X = (float*)(b + o_x), *xn = (float*)(b + o_xn), *qkv = (float*)(b + o_qkv), *q = (float*)(b + o_q);
   float *o = (float*)(b + o_o), *gu = (float*)(b + o_gu), *h = (float*)(b + o_h), *lg = (float*)(b + o_lg);
@@ -1280,16 +1313,19 @@ static int fwd_run(FDev *f, float rope_base, const int *ids, int n, float *logit
     for (int p0 = 0, i = 0; p0 < r && !rc; p0 += part, i++) {
       const int pr = r - p0 < part ? r - p0 : part;
       rc |= qhip_gemm_f32(0, FWD_CLS, xn + (size_t)p0 * dm, pr, f->dm, f->head, f->vocab, lg + p0 * V, NULL, pk);
-      rc = rc || qhip_dl_mark(g_fwd_dl, i);
+      rc = rc || qhip_dl_mark(dl, i);
     }
     if (!rc) qhip_dl_prefault(logits + (size_t)c0 * V, (size_t)r * V * 4);    // while the GPU is at the layers
     for (int p0 = 0, i = 0; p0 < r && !rc; p0 += part, i++) {
       const int pr = r - p0 < part ? r - p0 : part;
-      rc = qhip_dl_copy(g_fwd_dl, i, logits + ((size_t)c0 + p0) * V, lg + p0 * V, (size_t)pr * V * 4);
+      rc = qhip_dl_copy(dl, i, logits + ((size_t)c0 + p0) * V, lg + p0 * V, (size_t)pr * V * 4);
     }
-    if (qhip_dl_finish(g_fwd_dl)) rc = 1;
+    if (qhip_dl_finish(dl)) rc = 1;
   }
   if (qhip_sync()) rc = 1;
+  if (!rc) dl = atomic_exchange(&g_fwd_dl, dl);     // staging that has failed is not used again
+  qhip_dl_free(dl);
+  fwd_give(f, held);
   return rc;
 }
 

@@ -300,6 +300,55 @@ def test_f32_forward_two_passes_match_oracle(Q):
         ref.close()
 
 
+def test_f32_forwards_at_once_match_single_calls(Q):
+    """Forwards from several threads that overlap, on one model and on another:
+    every call's logits are those of the same call made alone."""
+    from concurrent.futures import ThreadPoolExecutor
+    refs = [O.FModel([2100, 96, 2, 2, 1, 48, 130, 320], 10000.0, seed=s) for s in (61, 62)]
+    gs = [gpu_model(Q, r, [2100, 96, 2, 2, 1, 48, 130, 320], 10000.0) for r in refs]
+    try:
+        work = [(i % 2 if k == 2 else 0, [(11 * j + i) % 2100 for j in range(rows)])
+                for k in range(3) for i, rows in enumerate((300, 70, 130, 257))]
+        alone = [gs[g].forward(ids).copy() for g, ids in work]
+        with ThreadPoolExecutor(4) as pool:
+            for _ in range(4):
+                got = list(pool.map(lambda w: gs[w[0]].forward(w[1]).copy(), work))
+                for a, b in zip(alone, got):
+                    assert np.array_equal(bits(a), bits(b))
+    finally:
+        for x in gs + refs:
+            x.close()
+
+
+def test_f32_forward_keeps_a_bounded_workspace(Q):
+    """What a long forward used (here 600 rows of 128256 logits, over 300 MB) is given
+    back when it ends, with a cache of the model alive; calls after it still match."""
+    import ctypes as C
+
+    def free_bytes():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert Q.lib().hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    cfg = [128256, 48, 1, 1, 1, 48, 32, 640]
+    ref = O.FModel(cfg, 10000.0, seed=8)
+    try:
+        g = gpu_model(Q, ref, cfg, 10000.0)
+        try:
+            few = g.forward([3, 128255, 7]).copy()
+            before = free_bytes()
+            L = g.forward([(97 * i + 3) % cfg[0] for i in range(600)])
+            assert before - free_bytes() < (32 << 20)
+            r = [ref.step((97 * i + 3) % cfg[0]).copy() for i in range(2)]
+            for i in range(2):
+                assert np.array_equal(bits(L[i]), bits(r[i]))
+            assert np.array_equal(bits(g.forward([3, 128255, 7])), bits(few))
+        finally:
+            g.close()
+    finally:
+        ref.close()
+
+
 def test_f32_forward_past_max_seq_matches_oracle(Q):
     """seq_len above the model's max_seq (the reference's forward has no such
     bound, llama.c:167-186): positions 16 .. 39 take RoPE tables made for the
