@@ -178,16 +178,19 @@ struct Stager {
   int next = 0;
 } g_up;
 
+// A large copy by up to four threads, this one among them; where no thread can be
+// started it takes what they would have.
 void par_copy(void *dst, const void *src, size_t n, size_t min_part = (size_t)8 << 20) {
-  const int parts = n >= 4 * min_part ? 4 : 1;
-  if (parts == 1) { memcpy(dst, src, n); return; }
-  std::vector<std::thread> th;
-  const size_t per = (n + parts - 1) / parts;
-  for (int i = 0; i < parts; i++) {
-    const size_t o = per * (size_t)i, c = o >= n ? 0 : (n - o < per ? n - o : per);
-    if (c) th.emplace_back([=] { memcpy((char *)dst + o, (const char *)src + o, c); });
+  const size_t per = n >= 4 * min_part ? (n + 3) / 4 : n;
+  std::thread th[3];
+  size_t o = 0;
+  int started = 0;
+  try {
+    for (; o + per < n; o += per, started++) th[started] = std::thread([=] { memcpy((char *)dst + o, (const char *)src + o, per); });
+  } catch (...) {
   }
-  for (auto &t : th) t.join();
+  memcpy((char *)dst + o, (const char *)src + o, n - o);
+  for (int i = 0; i < started; i++) th[i].join();
 }
 }  // namespace
 
@@ -250,13 +253,15 @@ struct Downloader {
   int next = 0;            // the buffer to empty first
 };
 
-// Wait for buffer b's copy and hand its bytes to their host destination.
+// Wait for buffer b's copy and hand its bytes to their host destination.  A copy whose
+// wait fails is dropped: the destination is the caller's again when its call returns.
 int dl_empty(Downloader *d, int b) {
-  if (!d->pend[b]) return 0;
+  const size_t n = d->pend[b];
+  if (!n) return 0;
+  d->pend[b] = 0;
   hipError_t e = hipEventSynchronize(d->ev[b]);
   if (e != hipSuccess) return fail("download wait", e);
-  par_copy(d->dst[b], d->buf[b], d->pend[b], (size_t)2 << 20);
-  d->pend[b] = 0;
+  par_copy(d->dst[b], d->buf[b], n, (size_t)2 << 20);
   return 0;
 }
 }  // namespace
