@@ -36,12 +36,12 @@ int         qhip_upload_begin(size_t chunk);
 int         qhip_upload(void *dst, const void *host_src, size_t n);
 int         qhip_upload_end(void);
 // Staged download of results of the library stream to pageable host memory, beside
-// the launches enqueued after them: mark i (0 .. qhip_dl_max_marks() - 1) names
+// the launches enqueued after them: mark i (0 .. QHIP_DL_MARKS - 1) names
 // what has been enqueued when it is set, copy(i) takes n bytes that were ready
 // there, finish waits until every byte has reached the host.
+#define QHIP_DL_MARKS 8
 void *qhip_dl_create(size_t chunk);
 void qhip_dl_free(void *h);
-int qhip_dl_max_marks(void);
 void qhip_dl_prefault(void *dst, size_t n);   // bring the destination's pages in (host work, no device call)
 int qhip_dl_mark(void *h, int i);
 int qhip_dl_copy(void *h, int i, void *dst, const void *src, size_t n);

@@ -243,11 +243,10 @@ int qhip_upload_end(void) {
 // beside the launches that follow the results on the library stream; the CPU
 // empties one buffer while the other is filled.
 namespace {
-constexpr int kDlMarks = 16;
 struct Downloader {
   hipStream_t stream = nullptr;
   void *buf[2] = {nullptr, nullptr};
-  hipEvent_t ev[2] = {nullptr, nullptr}, mark[kDlMarks] = {};
+  hipEvent_t ev[2] = {nullptr, nullptr}, mark[QHIP_DL_MARKS] = {};
   void *dst[2] = {nullptr, nullptr};
   size_t pend[2] = {0, 0}, chunk = 0;
   int next = 0;            // the buffer to empty first
@@ -274,7 +273,7 @@ void qhip_dl_free(void *h) {
     if (d->buf[b]) (void)hipHostFree(d->buf[b]);
     if (d->ev[b]) (void)hipEventDestroy(d->ev[b]);
   }
-  for (int i = 0; i < kDlMarks; i++)
+  for (int i = 0; i < QHIP_DL_MARKS; i++)
     if (d->mark[i]) (void)hipEventDestroy(d->mark[i]);
   if (d->stream) (void)hipStreamDestroy(d->stream);
   delete d;
@@ -289,7 +288,7 @@ void *qhip_dl_create(size_t chunk) {
     e = hipHostMalloc(&d->buf[b], chunk, hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d->ev[b], hipEventDisableTiming);
   }
-  for (int i = 0; i < kDlMarks && e == hipSuccess; i++) e = hipEventCreateWithFlags(&d->mark[i], hipEventDisableTiming);
+  for (int i = 0; i < QHIP_DL_MARKS && e == hipSuccess; i++) e = hipEventCreateWithFlags(&d->mark[i], hipEventDisableTiming);
   if (e != hipSuccess) {
     fail("download staging", e);
     (void)hipGetLastError();
@@ -311,9 +310,7 @@ void qhip_dl_prefault(void *dst, size_t n) {
 #endif
 }
 
-int qhip_dl_max_marks(void) { return kDlMarks; }
-
-// Mark the results enqueued so far on the library stream (i = 0 .. kDlMarks - 1).
+// Mark the results enqueued so far on the library stream (i = 0 .. QHIP_DL_MARKS - 1).
 int qhip_dl_mark(void *h, int i) {
   hipError_t e = hipEventRecord(static_cast<Downloader *>(h)->mark[i], g_stream);
   return e == hipSuccess ? 0 : fail("download mark", e);

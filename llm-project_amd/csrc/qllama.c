@@ -1300,15 +1300,22 @@ static int fwd_run(FDev *f, float rope_base, const int *ids, int n, float *logit
       rc |= qhip_swiglu_f32_rows(gu, r, f->dff, h);
       rc |= qhip_gemm_f32(1, FWD_CLS, h, r, f->dff, f->wd[l], f->dm, Xc, NULL, pk);
     }
-  // final norm and head (llama.c:182-183), in parts of whole 64-row tiles with about
-  // a staged copy of logits each: a part's logits go to the host while the next
-  // parts are computed
-  const int most = qhip_dl_max_marks();
+  // final norm and head (llama.c:182-183), in parts: a part's logits go to the host
+  // while the next parts are computed.  A part is an eighth of the rows, but no less
+  // than a staged copy, than 64 rows, and than 128 where 64 give the product fewer than
+  // 2.75 blocks a CU (under 45056 logits).  The copy is a kernel of the runtime's that
+  // slows the product beside it by about its own time, the more the fewer blocks the
+  // product has (64 rows of 32000: 155 us alone, 290 beside a copy of 149).  The whole
+  // call by rows a part, 1B-shaped layers, ms: 512 rows, four layers, of 32000 logits:
+  // 64 7.95, 128 7.46, 256 7.45, all 8.07; one layer, 64 and 128: of 40000 4.2 and 3.75,
+  // of 45000 4.25 and 4.13 (400 rows 3.54 and 3.60), of 49000 4.29 and 4.49; one layer
+  // of 32000: 1024 rows 64 8.9, 128 7.5, 256 7.3; 2048 rows 128 15.2, 256 14.8, 512 14.9.
   for (int c0 = 0; c0 < n && !rc; c0 += R) {
-    const int r = n - c0 < R ? n - c0 : R;
-    int part = (int)(FWD_DL_CHUNK / (V * 4)) / 64 * 64;
-    if (part < 64) part = 64;
-    if ((r + part - 1) / part > most) part = ((r + most - 1) / most + 63) / 64 * 64;
+    const int r = n - c0 < R ? n - c0 : R, chunk = (int)(FWD_DL_CHUNK / (V * 4)) / 64 * 64;
+    const int least = f->vocab < 45056 ? 128 : 64;
+    int part = ((r + QHIP_DL_MARKS - 1) / QHIP_DL_MARKS + 63) / 64 * 64;
+    if (part < least) part = least;
+    if (part < chunk) part = chunk;
     rc |= qhip_rmsnorm_f32_rows(X + (size_t)c0 * dm, r, f->dm, f->g_final, f->eps, xn);
     for (int p0 = 0, i = 0; p0 < r && !rc; p0 += part, i++) {
       const int pr = r - p0 < part ? r - p0 : part;

@@ -157,12 +157,13 @@ def test_f32_gemv_sees_its_own_panels_only(Q, pro, mode, K):
 
 
 @pytest.mark.parametrize("rows,dff,vocab", [(1, 33, 70), (5, 64, 17), (9, 100, 130), (40, 31, 64), (70, 95, 2100),
-                                            (300, 66, 16384)])
+                                            (300, 66, 16384), (130, 34, 16384), (300, 66, 40001)])
 def test_f32_forward_tile_edges_match_oracle(Q, rows, dff, vocab):
     """The many-row fp32 matmul where its tiles end: rows around a wave's and a
     block's (each of the row groups of 1, 2, 4 and 8 is taken by one of these),
     k rows past whole stages, batches and groups of four, column panels cut
-    short: every row bit for bit the oracle's step."""
+    short; and where the head's parts and the staged copies of their logits end
+    (a part of one copy and one of two rows, parts of three copies): every row bit for bit the oracle's step."""
     cfg = [vocab, 144, 1, 3, 1, 48, dff, 320]
     ref = O.FModel(cfg, 10000.0, seed=rows)
     try:
