@@ -162,7 +162,10 @@ void llama_decode_step(const LlamaModel *m, LlamaKV *kv, int token, Tensor *logi
 // 64 or 128 with at most 8 query heads per KV head, seq_len <= 16384 (max_seq
 // does not bound it); other head layouts replay decode steps, seq_len <= max_seq.
 // Uses the model's device copy if a cache holds one, else uploads one for the
-// call.  Ids outside [0, vocab) abort with a message.
+// call.  Calls may overlap in several threads.  Between calls a model keeps at most
+// 256 MiB of device workspace (freed with its last cache), the process 16 MiB of
+// pinned staging (freed with the last fp32 model).  Ids outside [0, vocab) abort
+// with a message.
 void llama_model_forward(const LlamaModel *m, const int *ids, int seq_len, Tensor *logits);
 
 // sampler.h:12-31.  Inside the reference's build this takes the place of

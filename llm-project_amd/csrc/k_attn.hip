@@ -1257,8 +1257,10 @@ __device__ __forceinline__ void mx_store4(__amdgpu_buffer_rsrc_t r, int off, flo
 // (smaller steps would fetch a line from L2 once for each of them).
 // Bound: a SIMD's issue of MFMAs and adds, which do not overlap (64.5 ns per 2048
 // products: 264 us at the 8B shape, 2048 rows).  Held to 4 waves per SIMD (128
-// registers): the issue rate rises with a SIMD's waves.  356 us at that shape (332 on
-// a cool card, under a kernel trace) and 20.1 at 333 rows of hd 64.
+// registers): the issue rate rises with a SIMD's waves.  373-382 -> 341-354 us at that
+// shape and 22.9 -> 19.9 at 333 rows of hd 64, timed in turn against q and K both from
+// memory a line at a time and each element's address and test formed on its own (about
+// 600 instructions a wave, many of them multiplies, after 4096 adds).
 template <int HD, int NP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_pf_scores_mx(const float *q, const float *kc, int R, int p0, int H,
                                                       int KVH, int max_seq, float scale, float *w, int Tp) {
@@ -1356,9 +1358,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // adds a lane per key: with NP = 16 the longest rows' waves, which bound the
 // kernel, carry half the adds of NP = 32).  Keys up to the block's first row's
 // last are seen by every pair: they go 8 a chunk, three chunks in flight, through
-// buffer loads whose position is one scalar (354 -> 347 us at the 8B shape, 2048
-// rows, 32.0 -> 29.8 at 333 rows of hd 64, against one chunk in flight and a 64-bit
-// address per load; two and four chunks the same).  Past them (at most rbq - 1 + 7 keys) a pair whose row ends
+// buffer loads (32.1 -> 29.8 us at 333 rows of hd 64 against one chunk in flight and
+// a 64-bit address per load; at the 8B shape, 2048 rows, no difference, 345-351 us
+// both; two and four chunks the same).  Past them (at most rbq - 1 + 7 keys) a pair whose row ends
 // before t supplies a zero weight, so its products are +-0 and its sums do not
 // move; should such a key's V value not be finite (0 * inf is NaN), that key
 // masks the products element by element instead.

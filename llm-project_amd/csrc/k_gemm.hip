@@ -601,11 +601,11 @@ int launch_pipe(const int8_t *A, const float *as, const int8_t *W, const float *
 // step's fragments, so its buffer takes the copies of step + NS, and the copies of
 // the next step, issued NS - 1 steps ago, have landed for the reads of that phase.
 // Limit: the compiler's hazard recognizer does not see the products inside the asm
-// blocks.  They follow one another without gaps (a block reads the sums only as the
-// products' own accumulators, for which the hardware waits), and the s_nops behind the
-// loop cover the last ones; but nothing else may read or move the sums between two
-// blocks: no operation on acc there, and no spill or copy of it (the accumulators and
-// fragments fit: the build's resource report shows no scratch for these kernels).
+// blocks.  The blocks read the sums only as accumulators, each last written three or
+// more products before, and the s_nops behind the loop cover the last ones; but nothing
+// else may read or move the sums between two blocks: no operation on acc there, and no
+// spill or copy of it (none in the assembly between the first product and the s_nops,
+// in any form; the residual 256 x 256 one spills 24 registers in its epilogue).
 // ---------------------------------------------------------------------------
 constexpr int DK = 128;
 
